@@ -45,9 +45,8 @@
 //   the running max is raised lazily (only when a tile exceeds it by more than
 //   2^8), so the O rescale is skipped on most tiles.
 // * Work items are ordered longest-first (causal tiles near the end of the
-//   sequence have the most keys) and mapped so that each XCD receives a
-//   contiguous range of (head group, query tile) items, keeping a KV head's
-//   tiles in one L2.
+//   sequence have the most keys), over all packed requests together, and dealt
+//   so that every XCD holds equal work and few KV heads share an L2.
 #include <algorithm>
 #include <type_traits>
 
@@ -64,6 +63,7 @@ namespace {
 constexpr int kBlockM = 32;  // queries per wavefront
 constexpr int kBlockN = 64;  // keys per LDS tile
 constexpr int kNumXcd = 8;
+constexpr int kLookupSeqs = 256;  // packed requests up to which items are looked up by rank (packed_tile)
 constexpr int kMaxUnits = 768;  // work units per group of a split launch (kernel-argument table)
 
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -73,8 +73,9 @@ typedef __attribute__((address_space(3))) v4i16_t lds_v4i16_t;
 // The fields the work-item decode reads come first: a workgroup's first
 // scalar loads of its arguments then share cache lines.
 struct GqaArgs {
-  int n_items;    // work items (workgroups with work)
-  int n_qtiles;   // query tiles per (sequence, head group)
+  int n_qtiles;   // query tiles per (sequence, head group); of the longest request when packed
+  int n_ranks;    // ranks of a group: its query tiles, or with the lookup a bound on all packed requests'
+  int lookup;     // packed requests: ranks are looked up (packed_tile)
   int n_hgroups;  // q_heads / hpw
   int hpw;        // query heads per workgroup
   int qpw;        // 32-query blocks per workgroup (hpw * qpw == 4)
@@ -85,7 +86,7 @@ struct GqaArgs {
   // unnormalised (o, running max, denominator) to `part`; gqa_combine_kernel
   // merges them.
   int n_split;    // 0: no split
-  int n_groups;   // sequences * head groups
+  int n_groups;   // sequences * head groups (with the lookup: head groups)
   int n_units;    // work units per group: n_qtiles + n_split
   int n_pad;      // n_units rounded up to a multiple of xcd_per_group
   int xcd_per_group;
@@ -220,6 +221,86 @@ __device__ __forceinline__ void store_rows(const GqaArgs& a, const f32x16_t (&o)
   }
 }
 
+// Rows [start, end) of packed request s, clamped to [0, T], so a malformed
+// offset table cannot move an access outside q/k/v/o.
+__device__ __forceinline__ void packed_bounds(const GqaArgs& a, int s, int* start, int* end) {
+  *start = min(max(a.cu[s], 0), a.seq_len);
+  *end = min(max(a.cu[s + 1], *start), a.seq_len);
+}
+
+// Sum of an int over the 64 lanes.
+__device__ __forceinline__ int wave_sum(int v) {
+  auto add = [&](auto m) {
+    float p, q;
+    fd_xor_pair<decltype(m)::value>(__uint_as_float(static_cast<uint32_t>(v)), p, q);
+    v = static_cast<int>(__float_as_uint(p) + __float_as_uint(q));
+  };
+  add(std::integral_constant<int, 1>{});
+  add(std::integral_constant<int, 2>{});
+  add(std::integral_constant<int, 4>{});
+  add(std::integral_constant<int, 8>{});
+  add(std::integral_constant<int, 16>{});
+  add(std::integral_constant<int, 32>{});
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+// The query tile of `rank` among the tiles of all packed requests, the tiles
+// with the larger index (the longer ones) first; false if there is none.  The
+// lengths are on the device only, so the host cannot build this table.  A lane
+// holds the tile counts of requests 64 c + lane, the number of tiles of index
+// >= t is one wavefront sum, and a binary search over t finds the rank's index
+// (8 sums at 8192 tokens).
+__device__ __forceinline__ bool packed_tile(const GqaArgs& a, int rank, int lane, int* seq, int* tile, int* start,
+                                            int* end) {
+  const int qspan = kBlockM * a.qpw;
+  constexpr int kPer = kLookupSeqs / 64;
+  int n[kPer], first[kPer], last[kPer];
+#pragma unroll
+  for (int c = 0; c < kPer; ++c) {
+    const int s = 64 * c + lane;
+    first[c] = last[c] = 0;
+    if (s < a.n_seqs) packed_bounds(a, s, &first[c], &last[c]);
+    n[c] = min((last[c] - first[c] + qspan - 1) / qspan, a.n_qtiles);
+  }
+  auto at_least = [&](int t) {
+    int m = 0;
+#pragma unroll
+    for (int c = 0; c < kPer; ++c) m += max(n[c] - t, 0);
+    return wave_sum(m);
+  };
+  if (rank >= at_least(0)) return false;
+  int lo = 0, hi = a.n_qtiles, after = 0;  // at_least(lo) > rank >= at_least(hi) == after
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    const int m = at_least(mid);
+    if (m > rank) {
+      lo = mid;
+    } else {
+      hi = mid;
+      after = m;
+    }
+  }
+  *tile = lo;
+  int k = rank - after;  // the k-th request with more than `lo` tiles
+  bool found = false;
+#pragma unroll
+  for (int c = 0; c < kPer; ++c) {
+    const uint64_t has = __builtin_amdgcn_ballot_w64(n[c] > lo);
+    const int before = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+        static_cast<uint32_t>(has >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(has), 0)));
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(n[c] > lo && before == k);
+    if (!found && hit != 0) {
+      const int at = __builtin_ctzll(hit);
+      *seq = 64 * c + at;
+      *start = __builtin_amdgcn_readlane(first[c], at);
+      *end = __builtin_amdgcn_readlane(last[c], at);
+      found = true;
+    }
+    k -= __builtin_popcountll(has);
+  }
+  return found;
+}
+
 template <int D, int KSPLIT>
 __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
   using C = Cfg<D, KSPLIT>;
@@ -238,6 +319,7 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
   const int nb = gridDim.x;
   const int b = blockIdx.x;
   int qtile, wgroup, part = -1;
+  int seq_start = 0, seq_end = a.seq_len;
   if (a.n_split > 0) {
     // Key split.  Block b runs on XCD b % 8; each group (one KV head's query
     // heads of one sequence) goes to xcd_per_group XCDs, which take every
@@ -254,26 +336,57 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
     qtile = code >> 2;
     part = (code & 3) - 1;
   } else {
-    // XCD-contiguous renumbering, longest tile first
-    const int item = (nb % kNumXcd == 0) ? (b % kNumXcd) * (nb / kNumXcd) + b / kNumXcd : b;
-    if (item >= a.n_items) return;
-    qtile = a.n_qtiles - 1 - item % a.n_qtiles;
-    wgroup = item / a.n_qtiles;
+    // Block b runs on XCD b % 8; the i-th block there takes the i-th longest of
+    // that XCD's share.  Query tiles come by rank, longest first: rank r of
+    // every group (a KV head's query heads of one sequence) is its tile
+    // n_qtiles - 1 - r; with the lookup a group is a head group and ranks run
+    // over the tiles of all packed requests together.  Per 8 ranks an XCD takes
+    // whole groups while there are 8 of them to deal, and every 8th item of the
+    // remaining ones, so all XCDs hold equal work at any moment and one L2 still
+    // sees few KV heads.  (Contiguous ranges of items per XCD, as before, gave
+    // one XCD the long half of a group and the next the short one, and left a
+    // long packed request's four head groups on two XCDs: B=1, T=8192, 16/4 x
+    // 128: 371 -> 295 us; four packed requests of 4177, 611, 8002 and 301
+    // tokens: 1142 -> 420 us.)
+    const int x = b % kNumXcd, i = b / kNumXcd;
+    const int full = a.n_groups / kNumXcd, rest = a.n_groups % kNumXcd;
+    int rank;
+    if (rest == 0) {
+      const int g = i / a.n_ranks;  // whole groups only: one after the other
+      rank = i - g * a.n_ranks;
+      wgroup = x * full + g;
+    } else if (full == 0) {
+      rank = b / rest;              // fewer groups than XCDs: the mixed form below, reduced
+      wgroup = b - rank * rest;
+      if (rank >= a.n_ranks) return;
+    } else {
+      const int blk = min(i / a.n_groups, a.n_ranks / kNumXcd);  // 8 ranks of an XCD: 8 * full + rest items
+      const int j = i - blk * a.n_groups;
+      const int cnt = min(kNumXcd, a.n_ranks - kNumXcd * blk);   // ranks in this block of them
+      if (j < cnt * full) {
+        const int r = j / full;
+        rank = kNumXcd * blk + r;
+        wgroup = x * full + (j - r * full);
+      } else {
+        const int L = (j - cnt * full) * kNumXcd + x;
+        if (L >= cnt * rest) return;
+        const int r = L / rest;
+        rank = kNumXcd * blk + r;
+        wgroup = kNumXcd * full + (L - r * rest);
+      }
+    }
+    if (a.lookup) {
+      int seq;
+      if (!packed_tile(a, rank, lane, &seq, &qtile, &seq_start, &seq_end)) return;
+      wgroup += seq * a.n_hgroups;
+    } else {
+      qtile = a.n_qtiles - 1 - rank;
+      if (a.cu != nullptr) packed_bounds(a, wgroup / a.n_hgroups, &seq_start, &seq_end);
+    }
   }
   const int hg = wgroup % a.n_hgroups;
   const int sidx = wgroup / a.n_hgroups;
-
-  int seq_start, seq_end, bidx;
-  if (a.cu != nullptr) {
-    // clamped to [0, T], so a malformed offset table cannot move an access outside q/k/v/o
-    seq_start = min(max(a.cu[sidx], 0), a.seq_len);
-    seq_end = min(max(a.cu[sidx + 1], seq_start), a.seq_len);
-    bidx = 0;
-  } else {
-    seq_start = 0;
-    seq_end = a.seq_len;
-    bidx = sidx;
-  }
+  const int bidx = a.cu == nullptr ? sidx : 0;
   const int qspan = kBlockM * a.qpw;
   const int q0 = seq_start + qtile * qspan;
   if (q0 >= seq_end) return;  // uniform over the workgroup
@@ -1072,6 +1185,8 @@ int gqa_launch(const void* q, const void* k, const void* v, void* out, const int
 
   const GqaShape g = gqa_shape(batch, q_heads, kv_heads, seq_len, n_seqs, max_seqlen, cu_seqlens != nullptr);
   GqaArgs a;
+  a.n_ranks = 0;
+  a.lookup = 0;
   a.q = static_cast<const uint16_t*>(q);
   a.k = static_cast<const uint16_t*>(k);
   a.v = static_cast<const uint16_t*>(v);
@@ -1095,21 +1210,38 @@ int gqa_launch(const void* q, const void* k, const void* v, void* out, const int
   a.n_qtiles = g.n_qtiles;
   a.n_hgroups = g.n_hgroups;
   FD_REQUIRE(g.items < 2147483647LL / 2, FD_ERR_INVALID_ARGUMENT, "fd_gqa_fwd: problem too large");
+  const bool varlen = cu_seqlens != nullptr;
   a.n_groups = g.n_hgroups * g.n_slots;
-  a.n_split = split_tiles(g.n_qtiles, g.items, cu_seqlens != nullptr, head_dim);
+  a.n_split = split_tiles(g.n_qtiles, g.items, varlen, head_dim);
   a.part = static_cast<float*>(workspace);
   if (a.n_split > 0 && (workspace == nullptr || !fd_aligned16(workspace) ||
                         workspace_bytes < split_bytes(a.n_groups, a.n_split, head_dim)))
     a.n_split = 0;  // no room for the halves: every tile runs whole
-  int64_t items = g.items;
+  int64_t nblocks;
   if (a.n_split > 0) {
     fill_units(a, kBlockM * g.qpw);
-    items = static_cast<int64_t>(a.n_groups) * a.n_pad;
+    const int64_t items = static_cast<int64_t>(a.n_groups) * a.n_pad;
+    nblocks = (items + kNumXcd - 1) / kNumXcd * kNumXcd;
+  } else {
+    int64_t ranks = g.n_qtiles;
+    if (varlen) {
+      // Packed requests hold at most `tight` tiles (each fills its tiles but for the
+      // last); dealt as a padded batch, n_qtiles each.  A workgroup pays about 0.6 us
+      // for the lookup and 1.5 us if it is empty: requests of like lengths (fewer than
+      // half of the padded tiles empty) and more than kLookupSeqs run as a padded batch.
+      const int64_t tight = seq_len / (kBlockM * g.qpw) + static_cast<int64_t>(n_seqs);
+      a.lookup = n_seqs <= kLookupSeqs && ranks * n_seqs > 2 * tight;
+      if (a.lookup) {
+        ranks = tight;
+        a.n_groups = g.n_hgroups;
+      }
+    }
+    a.n_ranks = static_cast<int>(ranks);
+    const int64_t full = a.n_groups / kNumXcd, rest = a.n_groups % kNumXcd, last = ranks % kNumXcd;
+    nblocks = kNumXcd * (ranks / kNumXcd * a.n_groups + last * full + (last * rest + kNumXcd - 1) / kNumXcd);
   }
-  a.n_items = static_cast<int>(items);
-  const int nblocks = static_cast<int>((items + kNumXcd - 1) / kNumXcd * kNumXcd);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  dim3 grid(nblocks);
+  dim3 grid(static_cast<unsigned>(nblocks));
   switch (head_dim) {
     case 64:
       hipLaunchKernelGGL((gqa_fwd_kernel<64, 2>), grid, dim3(Cfg<64, 2>::kThreads), 0, s, a);

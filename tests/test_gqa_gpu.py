@@ -200,6 +200,44 @@ def test_varlen_equals_per_request():
         assert (o[:, :, a:b].float() - ref).abs().max().item() <= ATOL
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,lengths", [
+    (16, 4, 128, [1]),
+    (16, 4, 128, [33, 0, 1, 2048, 32, 64, 1000]),           # equal and unequal tile counts, an empty request
+    (16, 4, 64, [(7 * i) % 91 for i in range(150)]),        # more requests than lanes
+    (12, 4, 128, [300, 129, 127, 513]),                     # 3 heads per group: 128-query tiles, 12 head groups
+    (9, 9, 64, [(31 * i) % 257 for i in range(65)]),        # 9 head groups: one more than XCDs
+    (4, 2, 64, [(13 * i) % 40 for i in range(255)] + [900]),  # the most requests that are looked up
+    (4, 2, 64, [(13 * i) % 40 for i in range(256)] + [900]),  # one more: dealt request by request
+    (4, 2, 64, [40 + (13 * i) % 40 for i in range(100)]),   # like lengths: the same
+    (8, 2, 256, [700, 65, 0, 31, 190]),
+])
+def test_every_tile_of_packed_requests_is_computed(Hq, Hkv, D, lengths):
+    """The rank -> (request, tile) lookup of packed requests and the dealing of items over the XCDs cover every
+    row exactly once: each request's rows equal the request alone (key split off, as a packed call runs)."""
+    from fastdecisions_amd.native_gqa_kernel import native_gqa_attention
+    cu = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    T = int(cu[-1])
+    announce(f"gqa packed {Hq}/{Hkv}x{D} n={len(lengths)} T={T}")
+    q, k, v = model_layout(1, Hq, Hkv, T, D, 1500 + T, D ** -0.5)
+    o = native_gqa_attention(q, k, v, cu_seqlens=torch.from_numpy(cu).cuda(), max_seqlen=max(lengths))
+    for a, b in zip(cu[:-1], cu[1:]):
+        if b > a:
+            alone = native_gqa_attention(q[:, :, a:b], k[:, :, a:b], v[:, :, a:b], key_split=False)
+            assert torch.equal(o[:, :, a:b], alone), (a, b)
+    a, b = max(zip(cu[:-1], cu[1:]), key=lambda s: s[1] - s[0])
+    err = (o[:, :, a:b].float() - sdpa_fp32(q[:, :, a:b], k[:, :, a:b], v[:, :, a:b])).abs().max().item()
+    assert err <= ATOL, err
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T,D", [(3, 16, 4, 300, 128), (9, 4, 4, 33, 64), (40, 2, 1, 20, 64), (1, 28, 7, 65, 128)])
+def test_padded_batches_with_groups_that_do_not_divide_the_xcds(B, Hq, Hkv, T, D):
+    from fastdecisions_amd.native_gqa_kernel import native_gqa_attention
+    announce(f"gqa padded B={B} {Hq}/{Hkv}x{D} T={T}")
+    q, k, v = model_layout(B, Hq, Hkv, T, D, 1600 + T, 1.0)
+    err = (native_gqa_attention(q, k, v).float() - sdpa_fp32(q, k, v)).abs().max().item()
+    assert err <= ATOL, err
+
+
 @pytest.mark.parametrize("Hq,Hkv,T,D", [(16, 4, 2048, 128), (16, 4, 700, 64), (8, 2, 1024, 256)])
 def test_rows_do_not_depend_on_the_batch(Hq, Hkv, T, D):
     """A request's rows are bit-identical alone (B=1) and in padded batches of 2 and 5 sequences
