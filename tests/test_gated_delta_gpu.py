@@ -243,3 +243,28 @@ def test_rows_do_not_depend_on_the_batch(oracle, gd, T, hk, hv, B):
     ref, _ = gd.chunked(_np(q[:B]), _np(k[:B]), _np(v[:B]), g[:B].numpy(), _np(beta[:B]),
                         initial_state=s0[:B].numpy())
     _check(oracle, to_bits(out), ref, f"B={B} T={T} hv={hv}")
+
+
+@pytest.mark.parametrize("hk,hv,lengths", [
+    (16, 16, [0, 5, 64, 65, 0, 1000, 1]),                 # empty requests first, between and chunk-sized ones
+    (1, 3, [130, 0, 700]),                                # units that do not fill the XCDs
+    (1, 2, [(7 * i) % 71 for i in range(1030)]),          # more requests than threads of the table
+    (1, 1, [64] * 1024),
+])
+def test_packed_requests_equal_the_same_requests_alone(hk, hv, lengths):
+    """Chunk table, longest-first order and XCD dealing: every packed request's rows and final state equal the
+    request's own, bit for bit."""
+    T = sum(lengths)
+    announce(f"gated delta packed hk={hk} hv={hv} n={len(lengths)} T={T}")
+    q, k, v, g, beta = (t.cuda() for t in _inputs(T, hk, hv, 77))
+    cu = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    rule = _rule()
+    out, final = rule(q, k, v, g, beta, use_qk_l2norm_in_kernel=True, output_final_state=True,
+                      cu_seqlens=torch.from_numpy(cu).cuda())
+    for i, (a, b) in enumerate(zip(cu[:-1], cu[1:])):
+        if b == a:
+            assert not final[i].any()
+            continue
+        alone, state = rule(*(t[:, a:b].contiguous() for t in (q, k, v, g, beta)), use_qk_l2norm_in_kernel=True,
+                            output_final_state=True)
+        assert torch.equal(out[:, a:b], alone) and torch.equal(final[i], state[0]), (i, a, b)
