@@ -408,13 +408,12 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
   const float c = a.scale_log2;
 
   // Q^T as MFMA B operand: lane supplies Q[qpos][16kk + 8*half + 0..7].
+  // The loops issue their copies as asm and count them themselves; the compiler,
+  // which does not see them, must not be left with loads of its own to wait for.
+  // So Q is read with asm too, before any copy, and the prologue's copy wait
+  // covers it.  Rows past the end read the last row and are zeroed after that wait.
   bf16x8_t qf[D / 16];
-  if constexpr (KSPLIT == 1) {
-    // The head_dim-256 loop issues its copies and LDS reads as asm and counts
-    // them itself; the compiler, which does not see them, must not be left
-    // with loads of its own to wait for inside the loop.  So Q is read with
-    // asm too, before any copy, and the prologue's copy wait covers it.  Rows
-    // past the end read the last row and are zeroed after that wait.
+  {
     typedef unsigned u32x4q_t __attribute__((ext_vector_type(4)));
     const int qrow = qvalid ? qpos : seq_end - 1;
     const uint16_t* qp = qbase + qrow * a.qs[2] + half * 8;
@@ -424,14 +423,14 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
       asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(raw) : "v"(qp), "i"(kk * 32) : "memory");
       qf[kk] = __builtin_bit_cast(bf16x8_t, raw);
     }
-  } else {
+  }
+  auto q_arrived = [&]() {
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk) {
-      uint4 u = make_uint4(0u, 0u, 0u, 0u);
-      if (qvalid) u = *reinterpret_cast<const uint4*>(qbase + qpos * a.qs[2] + kk * 16 + half * 8);
-      qf[kk] = as_bf16x8(u);
+      asm volatile("" : "+v"(qf[kk]));
+      if (!qvalid) qf[kk] = bf16x8_t{};
     }
-  }
+  };
 
   const int kend = min(q0 + qspan, seq_end);
   const int nt_all = (kend - seq_start + kBlockN - 1) / kBlockN;
@@ -455,109 +454,14 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
     const int slot = (i * C::kWaves + wave) * 64 + lane;
     return ((slot % CR) ^ swz_v<CR>(slot / CR)) * 8;
   };
-  // K A operand: lane reads row (kh*kBlocks + bl)*32 + sigma(col), logical chunk 2kk + half.
-  // V^T A operand: two transposing reads per (dim block, 16-key slice).
-  // With two wavefronts per SIMD the byte offsets fit in registers and are
-  // computed once; the 4-wavefront head_dim-256 variant recomputes them.
   const int grp = lane >> 4;
   const int li = lane & 15;
-  auto k_off_calc = [&](int bl, int kk) {
-    const int row = (kh * C::kBlocks + bl) * 32 + sigma(col);
-    return row * CR * 16 + (((2 * kk + half) ^ swz_k<CR>(row)) * 16);
-  };
-  auto v_off_calc = [&](int db, int cs, int r2) {
-    const int dim = db * 32 + 16 * (grp & 1) + 4 * (li & 3);
-    const int row = ((kh * C::kBlocks) * 2 + cs) * 16 + 8 * (grp >> 1) + 4 * r2 + (li >> 2);
-    return row * CR * 16 + (((dim >> 3) ^ swz_v<CR>(row)) * 16) + (dim & 7) * 2;
-  };
-  constexpr bool kHoist = KSPLIT > 1;
-  int k_rd[kHoist ? C::kBlocks : 1][kHoist ? D / 16 : 1];
-  int v_rd[kHoist ? D / 32 : 1][kHoist ? 2 * C::kBlocks : 1][2];
-  if constexpr (kHoist) {
-#pragma unroll
-    for (int bl = 0; bl < C::kBlocks; ++bl)
-#pragma unroll
-      for (int kk = 0; kk < D / 16; ++kk) k_rd[bl][kk] = k_off_calc(bl, kk);
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int cs = 0; cs < 2 * C::kBlocks; ++cs)
-#pragma unroll
-        for (int r2 = 0; r2 < 2; ++r2) v_rd[db][cs][r2] = C::kStages * C::kTileBytes + v_off_calc(db, cs, r2);
-  }
-  int cp_krel[kHoist ? C::kLoads : 1], cp_vrel[kHoist ? C::kLoads : 1];
-  if constexpr (kHoist) {
-#pragma unroll
-    for (int i = 0; i < C::kLoads; ++i) {
-      cp_krel[i] = cp_row(i) * static_cast<int>(a.ks[2]) + cp_koff(i);
-      cp_vrel[i] = cp_row(i) * static_cast<int>(a.vs[2]) + cp_voff(i);
-    }
-  }
-  auto k_off = [&](int bl, int kk) {
-    if constexpr (kHoist) return k_rd[bl][kk]; else return k_off_calc(bl, kk);
-  };
-  // V^T operand address in stage BUF: the hoisted offsets include the V region's
-  // base, so the stage offset (< 64 KiB) is the read's immediate
-  auto v_addr = [&](int BUF, int db, int cs, int r2) -> const unsigned char* {
-    if constexpr (kHoist) return smem + BUF * C::kTileBytes + v_rd[db][cs][r2];
-    else return v_lds + BUF * C::kTileBytes + v_off_calc(db, cs, r2);
-  };
-
-  // rows past the end of the sequence re-read its last row: finite data the mask discards
-  auto issue_tile = [&](int t, int buf) {
-    const int ks0 = seq_start + (tb + t) * kBlockN;
-    unsigned char* kt = k_lds + buf * C::kTileBytes;
-    unsigned char* vt = v_lds + buf * C::kTileBytes;
-    const uint16_t* kg = kbase + ks0 * a.ks[2];
-    const uint16_t* vg = vbase + ks0 * a.vs[2];
-    const bool full = ks0 + kBlockN <= seq_end;
-    const int last = seq_end - 1 - ks0;  // last valid row of this tile
-#pragma unroll
-    for (int i = 0; i < C::kLoads; ++i) {
-      const int blk = i * C::kWaves + wave;
-      int krel, vrel;
-      if (full) {
-        krel = kHoist ? cp_krel[i] : cp_row(i) * static_cast<int>(a.ks[2]) + cp_koff(i);
-        vrel = kHoist ? cp_vrel[i] : cp_row(i) * static_cast<int>(a.vs[2]) + cp_voff(i);
-      } else {
-        const int r = cp_row(i) < last ? cp_row(i) : last;
-        krel = r * static_cast<int>(a.ks[2]) + cp_koff(i);
-        vrel = r * static_cast<int>(a.vs[2]) + cp_voff(i);
-      }
-      // uniform tile base + 32-bit per-lane byte offset (scalar-base addressing)
-      const void* ksrc = reinterpret_cast<const unsigned char*>(kg) + static_cast<uint32_t>(krel) * 2u;
-      const void* vsrc = reinterpret_cast<const unsigned char*>(vg) + static_cast<uint32_t>(vrel) * 2u;
-      __builtin_amdgcn_global_load_lds(ksrc, (lds_void_t*)(kt + blk * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(vsrc, (lds_void_t*)(vt + blk * 1024), 16, 0, 0);
-    }
-  };
 
   f32x16_t o[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) o[db] = f32x16_t{};
   float m_run = -__builtin_inff();  // running max (log2-scaled units), may lag the true max by <= 8
   float l_run = 0.0f;               // this lane's partial denominator
-
-  constexpr int kPerTile = 2 * C::kLoads;  // VMEM instructions per thread of one issue_tile
-
-  // S^T for this wavefront's 32-key block(s) of the tile in LDS stage BUF
-  auto scores = [&](int BUF, f32x16_t (&s)[C::kBlocks]) {
-    const unsigned char* kt = k_lds + BUF * C::kTileBytes;
-#pragma unroll
-    for (int bl = 0; bl < C::kBlocks; ++bl) {
-      s[bl] = f32x16_t{};
-      constexpr int kGroup = D / 16 < 8 ? D / 16 : 8;  // operand reads issued ahead of their MFMAs
-#pragma unroll
-      for (int k0 = 0; k0 < D / 16; k0 += kGroup) {
-        bf16x8_t kf[kGroup];
-#pragma unroll
-        for (int kk = 0; kk < kGroup; ++kk) kf[kk] = *reinterpret_cast<const bf16x8_t*>(kt + k_off(bl, k0 + kk));
-#pragma unroll
-        for (int kk = 0; kk < kGroup; ++kk)
-          s[bl] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk], qf[k0 + kk], s[bl], 0, 0, 0);
-      }
-    }
-  };
 
   // causal / end-of-sequence mask of tile t, on diagonal and tail tiles only
   auto mask = [&](int t, f32x16_t (&s)[C::kBlocks]) {
@@ -573,124 +477,230 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
     }
   };
 
-  // O = alpha O + V^T · P^T with V in stage BUF: the V^T A operand of each
-  // 16-key slice comes from two transposing reads of the row-major V tile
-  // (keys +0..3 and +4..7)
-  auto accumulate = [&](int BUF, const bf16x8_t (&pb)[2 * C::kBlocks], float alpha, bool grow_any) {
-    if (grow_any) {
-#pragma unroll
-      for (int db = 0; db < D / 32; ++db) o[db] *= alpha;
-    }
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db) {
-#pragma unroll
-      for (int cs = 0; cs < 2 * C::kBlocks; ++cs) {
-        const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)v_addr(BUF, db, cs, 0));
-        const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)v_addr(BUF, db, cs, 1));
-        const short __attribute__((ext_vector_type(8))) vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vv), pb[cs], o[db], 0, 0, 0);
-      }
-    }
-  };
-
   if constexpr (C::kPipe) {
-    // Prologue: tiles 0..2 in flight, wait for tiles 0 and 1, scores of tile 0.
-    issue_tile(0, 0);
-    if (ntiles > 1) issue_tile(1, 1);
-    if (ntiles > 2) {
-      issue_tile(2, 2);
-      __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(kPerTile));
-    } else {
-      __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(0));
+    // Step t runs in two phases with one barrier between them:
+    //   A: the score MFMAs of tile t+1, the second half of tile t's softmax
+    //      between them, and the reads of tile t's V operands;
+    //   B: the P·V MFMAs of tile t, the mask, maximum and first half of tile
+    //      t+1's softmax between them, and the reads of tile t+2's K operands.
+    // A wavefront's softmax costs as many issue cycles as its MFMAs (per step
+    // 63 VALU instructions and 17 exps, about 520, against 16 x 32), so half of
+    // it belongs to each MFMA phase: with all of it under the scores, the two
+    // wavefronts of a SIMD, which pass the barrier together, left the matrix
+    // core idle half of that phase and the VALU idle during P·V (@GQA@).
+    // Every operand is read a phase before its MFMA.
+    //
+    // LDS: a step copies tile t+3 into the stage tile t-1 left: its V operands
+    // had arrived (lgkmcnt 0) in every wavefront before the last barrier.  The
+    // barrier waits for all copies but this step's: tile t+2, whose K operands
+    // phase B reads, has landed.  The copies are asm: seen by the compiler, they
+    // would make it wait for them before every LDS read.
+    static_assert(C::kBlocks == 1, "the pipelined step takes one 32-key block per wavefront");
+    constexpr int kSteps = D / 16;   // score MFMAs per tile, and P·V MFMAs: (D / 32) O blocks x 2 key slices
+    constexpr int kNdb = D / 32;
+    constexpr int kPer = 8 / kSteps;  // softmax pieces per MFMA
+    constexpr int kPerTile = 2 * C::kLoads;  // copy instructions per thread of one tile
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_t*)smem));
+    // K A operand: row kh*32 + sigma(col), logical chunk 2kk + half
+    int k_rd[kSteps];
+#pragma unroll
+    for (int kk = 0; kk < kSteps; ++kk) {
+      const int row = kh * 32 + sigma(col);
+      k_rd[kk] = row * CR * 16 + (((2 * kk + half) ^ swz_k<CR>(row)) * 16);
     }
-    __syncthreads();
-    f32x16_t sA[C::kBlocks], sB[C::kBlocks];
-    scores(0, sA);
-
-    // Step t (stage BUF = t % 4): tile t+3 is issued into the stage tile t-1
-    // left (every wavefront passed the previous step's barrier); the softmax
-    // of tile t and the scores of tile t+1 (complete since the previous step)
-    // are independent, so their VALU and MFMA work can interleave.  At the
-    // end only tile t+3 may still be in flight: tile t+2, which the next
-    // step's scores read, has landed, and the barrier makes it visible.  The
-    // last step's scores read a stale stage and are discarded.
-    auto step = [&](int t, int BUF, f32x16_t (&sc)[C::kBlocks], f32x16_t (&sn)[C::kBlocks]) {
-      static_assert(C::kBlocks == 1, "the pipelined step takes one 32-key block per wavefront");
-      const bool issued = t + 3 < ntiles;
-      if (issued) issue_tile(t + 3, (BUF + 3) & 3);
-      mask(t, sc);
-      // The next tile's scores are a chain of D/16 dependent MFMAs; after each
-      // one the wavefront issues one piece of this tile's softmax (8 pieces),
-      // which runs while the MFMA does.  sched_barrier keeps the pieces apart.
-      constexpr int kSteps = D / 16;
-      constexpr int kPer = 8 / kSteps;  // softmax pieces per MFMA
-      const unsigned char* ktn = k_lds + ((BUF + 1) & 3) * C::kTileBytes;
-      float mx = -__builtin_inff(), alpha = 1.0f, m_sub = 0.0f, psum = 0.0f;
-      bool grow = false;
-      f32x8_t pv[2];
-      bf16x8_t pb[2];
-      auto piece = [&](int k) {
-        if (k == 0) {
+    // V^T A operand of O block db: two transposing reads (keys +0..3 and +4..7) per
+    // 16-key slice; the swizzle depends on row & 3 alone, so slices and row halves
+    // are immediates
+    int v_rd[kNdb];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[0][r]);
-        } else if (k == 1) {
-          mx = half_max(mx) * c;
-          grow = mx > m_run + 8.0f;
-          const float m_new = grow ? mx : m_run;
-          alpha = grow ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
-          m_sub = (m_new == -__builtin_inff()) ? 0.0f : m_new;  // fully masked so far: p = 0
-          m_run = m_new;
-        } else if (k < 6) {
-          const int r0 = 4 * (k - 2);  // scores r0 .. r0 + 3
+    for (int db = 0; db < kNdb; ++db) {
+      const int dim = db * 32 + 16 * (grp & 1) + 4 * (li & 3);
+      const int row = kh * 32 + 8 * (grp >> 1) + (li >> 2);
+      v_rd[db] = C::kStages * C::kTileBytes + row * CR * 16 + (((dim >> 3) ^ swz_v<CR>(row)) * 16) + (dim & 7) * 2;
+    }
+    int cp_krel[C::kLoads], cp_vrel[C::kLoads];
 #pragma unroll
-          for (int r = r0; r < r0 + 4; ++r) {
-            float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[0][r], c, -m_sub));
-            asm volatile("" : "+v"(p));  // computed here, not sunk towards its use in P·V
-            psum += p;
-            pv[r >> 3][r & 7] = p;
-          }
-        } else if (k == 6) {
-          pb[0] = __builtin_convertvector(pv[0], bf16x8_t);
-          pb[1] = __builtin_convertvector(pv[1], bf16x8_t);
-          asm volatile("" : "+v"(pb[0]), "+v"(pb[1]));
-        } else {
-          l_run = l_run * alpha + psum;
-          asm volatile("" : "+v"(l_run));
+    for (int i = 0; i < C::kLoads; ++i) {
+      cp_krel[i] = cp_row(i) * static_cast<int>(a.ks[2]) + cp_koff(i);
+      cp_vrel[i] = cp_row(i) * static_cast<int>(a.vs[2]) + cp_voff(i);
+    }
+    auto copy_tile = [&](int t, int buf) {
+      const int ks0 = seq_start + t * kBlockN;
+      const uint16_t* kg = kbase + ks0 * a.ks[2];
+      const uint16_t* vg = vbase + ks0 * a.vs[2];
+      const int last = seq_end - 1 - ks0;  // rows past the end re-read the last row: finite data the mask discards
+      const bool full = last >= kBlockN - 1;
+#pragma unroll
+      for (int i = 0; i < C::kLoads; ++i) {
+        int krel = cp_krel[i], vrel = cp_vrel[i];
+        if (!full) {
+          const int r = min(cp_row(i), last);
+          krel = r * static_cast<int>(a.ks[2]) + cp_koff(i);
+          vrel = r * static_cast<int>(a.vs[2]) + cp_voff(i);
         }
-      };
-      // All of the next tile's K operands are read before the chain: the
-      // compiler then waits once per tile for them (read one MFMA ahead, it
-      // waited at every MFMA for the read just issued); 38.6 -> 38.1 us at B=1.
-      sn[0] = f32x16_t{};
-      bf16x8_t kfa[kSteps];
-#pragma unroll
-      for (int kk = 0; kk < kSteps; ++kk) kfa[kk] = *reinterpret_cast<const bf16x8_t*>(ktn + k_off(0, kk));
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int kk = 0; kk < kSteps; ++kk) {
-        sn[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfa[kk], qf[kk], sn[0], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) piece(kk * kPer + j);
-        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t kl = lds0 + static_cast<uint32_t>(buf * C::kTileBytes + (i * C::kWaves + wave) * 1024);
+        const uint32_t vl = kl + static_cast<uint32_t>(C::kStages * C::kTileBytes);
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :: "v"(static_cast<uint32_t>(krel) * 2u), "s"(kg), "s"(kl) : "memory", "m0");
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :: "v"(static_cast<uint32_t>(vrel) * 2u), "s"(vg), "s"(vl) : "memory", "m0");
       }
-      const bool grow_any = __builtin_amdgcn_ballot_w64(grow) != 0;
-      accumulate(BUF, pb, alpha, grow_any);
-      if (issued)
+    };
+
+    f32x16_t sA[1], sB[1];
+    bf16x8_t kf[kSteps];                // K operands of the next tile
+    v4i16_t vlo[kSteps], vhi[kSteps];   // V operands of this tile, MFMA i: slice i / kNdb, O block i % kNdb
+    float p[16];                        // P of the tile whose softmax is under way
+    float alpha = 1.0f, m_sub = 0.0f, psum = 0.0f, mx = 0.0f;
+    bool grow = false;
+
+    auto read_k = [&](int BUF, int kk) {
+      kf[kk] = *reinterpret_cast<const bf16x8_t*>(k_lds + BUF * C::kTileBytes + k_rd[kk]);
+    };
+    auto read_v = [&](int BUF, int i) {
+      const unsigned char* vt = smem + BUF * C::kTileBytes + v_rd[i % kNdb] + (i / kNdb) * 16 * CR * 16;
+      vlo[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)vt);
+      vhi[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(vt + 4 * CR * 16));
+    };
+    // p of the scores r0 and r0 + 1, summed in order
+    auto exps = [&](const f32x16_t& s, int r0) {
+#pragma unroll
+      for (int r = r0; r < r0 + 2; ++r) {
+        p[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -m_sub));
+        asm volatile("" : "+v"(p[r]));  // computed here, not sunk towards its use in P·V
+        psum += p[r];
+      }
+    };
+    // softmax of a tile, first half: pieces 1 .. 6
+    auto head = [&](int k, const f32x16_t& s) {
+      if (k == 1) {
+        mx = -__builtin_inff();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+      } else if (k == 2) {
+        mx = half_max(mx) * c;
+        grow = mx > m_run + 8.0f;
+        const float m_new = grow ? mx : m_run;
+        alpha = grow ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
+        m_sub = (m_new == -__builtin_inff()) ? 0.0f : m_new;  // fully masked so far: p = 0
+        m_run = m_new;
+        psum = 0.0f;
+      } else if (k >= 3 && k < 7) {
+        exps(s, 2 * (k - 3));
+      }
+    };
+    // second half: pieces 0 .. 6
+    bf16x8_t pb[2];
+    auto tail = [&](int k, const f32x16_t& s) {
+      if (k < 4) {
+        exps(s, 8 + 2 * k);
+      } else if (k == 4) {
+        pb[0] = __builtin_convertvector(f32x8_t{p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7]}, bf16x8_t);
+        asm volatile("" : "+v"(pb[0]));
+      } else if (k == 5) {
+        pb[1] = __builtin_convertvector(f32x8_t{p[8], p[9], p[10], p[11], p[12], p[13], p[14], p[15]}, bf16x8_t);
+        asm volatile("" : "+v"(pb[1]));
+      } else if (k == 6) {
+        l_run = l_run * alpha + psum;
+        asm volatile("" : "+v"(l_run));
+      }
+    };
+    auto wait_copies = [&](bool in_flight) {
+      if (in_flight)
         __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(kPerTile));
       else
         __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(0));
-      __syncthreads();
     };
+
+    // Prologue: tiles 0..2 in flight, tiles 0 and 1 landed; scores of tile 0 and the head of its softmax.
+    copy_tile(0, 0);
+    if (ntiles > 1) copy_tile(1, 1);
+    if (ntiles > 2) copy_tile(2, 2);
+    wait_copies(ntiles > 2);
+    q_arrived();  // the Q loads are older than every copy
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < kSteps; ++kk) read_k(0, kk);
+    sA[0] = f32x16_t{};
+#pragma unroll
+    for (int kk = 0; kk < kSteps; ++kk) sA[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk], qf[kk], sA[0], 0, 0, 0);
+#pragma unroll
+    for (int kk = 0; kk < kSteps; ++kk) read_k(1, kk);
+    mask(0, sA);
+#pragma unroll
+    for (int k = 1; k < 8; ++k) head(k, sA[0]);
+
+    // BUF = t % 4; LAST: no tile t+1
+    auto step = [&](auto last_c, int t, int BUF, f32x16_t (&sc)[1], f32x16_t (&sn)[1]) {
+      constexpr bool LAST = decltype(last_c)::value;
+      const bool issued = !LAST && t + 3 < ntiles;
+      if (issued) copy_tile(t + 3, (BUF + 3) & 3);
+      // ---- phase A
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!LAST) {
+        sn[0] = f32x16_t{};
+#pragma unroll
+        for (int kk = 0; kk < kSteps; ++kk) {
+          sn[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk], qf[kk], sn[0], 0, 0, 0);
+          // two V operands behind each MFMA of the first half: the K operands make room
+          constexpr int kFirst = kSteps > 4 ? 1 : 0;
+          if (kk >= kFirst && kk < kFirst + kSteps / 2) {
+            read_v(BUF, 2 * (kk - kFirst));
+            read_v(BUF, 2 * (kk - kFirst) + 1);
+          }
+#pragma unroll
+          for (int j = 0; j < kPer; ++j) tail(kk * kPer + j, sc[0]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i) read_v(BUF, i);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) tail(k, sc[0]);
+      }
+      // O takes tile t's rescale here: phase B moves alpha on to tile t+1
+      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+#pragma unroll
+        for (int db = 0; db < kNdb; ++db) o[db] *= alpha;
+      }
+      if constexpr (!LAST) {
+        wait_copies(issued);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the V operands have arrived
+        __syncthreads();
+        mask(t + 1, sn);
+      }
+      // ---- phase B
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kSteps; ++i) {
+        const short __attribute__((ext_vector_type(8))) vv = {vlo[i][0], vlo[i][1], vlo[i][2], vlo[i][3],
+                                                              vhi[i][0], vhi[i][1], vhi[i][2], vhi[i][3]};
+        o[i % kNdb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vv), pb[i / kNdb],
+                                                              o[i % kNdb], 0, 0, 0);
+        if constexpr (!LAST) {
+          read_k((BUF + 2) & 3, i);
+#pragma unroll
+          for (int j = 0; j < kPer; ++j) head(i * kPer + j, sn[0]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    const std::false_type mid{};
+    const std::true_type last{};
+    const int n1 = ntiles - 1;
     int t = 0;
-    for (; t + 4 <= ntiles; t += 4) {
-      step(t, 0, sA, sB);
-      step(t + 1, 1, sB, sA);
-      step(t + 2, 2, sA, sB);
-      step(t + 3, 3, sB, sA);
+    for (; t + 4 <= n1; t += 4) {
+      step(mid, t, 0, sA, sB);
+      step(mid, t + 1, 1, sB, sA);
+      step(mid, t + 2, 2, sA, sB);
+      step(mid, t + 3, 3, sB, sA);
     }
-    if (t < ntiles) step(t, 0, sA, sB);
-    if (t + 1 < ntiles) step(t + 1, 1, sB, sA);
-    if (t + 2 < ntiles) step(t + 2, 2, sA, sB);
+    if (t < n1) step(mid, t, 0, sA, sB);
+    if (t + 1 < n1) step(mid, t + 1, 1, sB, sA);
+    if (t + 2 < n1) step(mid, t + 2, 2, sA, sB);
+    if (n1 & 1) sA[0] = sB[0];
+    step(last, n1, n1 & 3, sA, sB);
+    __syncthreads();  // every wavefront's LDS reads are done: the merge reuses the stages
   } else if constexpr (KSPLIT == 1) {
     // head_dim 256: one wavefront per SIMD (4 per workgroup), each owning one
     // head's 32 queries.  The wavefront walks the keys in 32-key blocks (block
@@ -773,11 +783,7 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
     copy_tile(0, true);
     if (ntiles > 1) __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(2 * C::kLoads));
     else __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(C::kLoads));
-#pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {  // the Q loads (older than every copy) have completed
-      asm volatile("" : "+v"(qf[kk]));
-      if (!qvalid) qf[kk] = bf16x8_t{};
-    }
+    q_arrived();  // the Q loads are older than every copy
     __syncthreads();
     f32x16_t S[2];   // scores of block b in S[b & 1]
     bf16x8_t P[2][2];  // P of block b in P[b & 1] (two 16-key slices)
