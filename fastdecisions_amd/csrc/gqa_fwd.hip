@@ -442,7 +442,6 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
   // 0..S-1]; K and V reads each use one base register plus an immediate
   // stage offset (< 64 KiB), the loop being unrolled by the stage count.
   unsigned char* const k_lds = smem;
-  unsigned char* const v_lds = smem + C::kStages * C::kTileBytes;
   // global -> LDS copies: copy i of this lane moves 16-byte chunk `slot` of a
   // tile (row = slot / CR, physical chunk = slot % CR, global chunk unswizzled)
   auto cp_row = [&](int i) { return ((i * C::kWaves + wave) * 64 + lane) / CR; };
@@ -462,20 +461,6 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
   for (int db = 0; db < D / 32; ++db) o[db] = f32x16_t{};
   float m_run = -__builtin_inff();  // running max (log2-scaled units), may lag the true max by <= 8
   float l_run = 0.0f;               // this lane's partial denominator
-
-  // causal / end-of-sequence mask of tile t, on diagonal and tail tiles only
-  auto mask = [&](int t, f32x16_t (&s)[C::kBlocks]) {
-    const int kb0 = seq_start + (tb + t) * kBlockN + kh * C::kBlocks * 32;  // first key of this wavefront's part
-    if (kb0 + C::kBlocks * 32 - 1 > qw0 || kb0 + C::kBlocks * 32 > seq_end) {
-#pragma unroll
-      for (int bl = 0; bl < C::kBlocks; ++bl)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kb0 + bl * 32 + (r >> 3) * 16 + half * 8 + (r & 7);
-          if (key > qpos || key >= seq_end) s[bl][r] = -__builtin_inff();
-        }
-    }
-  };
 
   if constexpr (C::kPipe) {
     // Step t runs in two phases with one barrier between them:
@@ -524,17 +509,18 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
       cp_krel[i] = cp_row(i) * static_cast<int>(a.ks[2]) + cp_koff(i);
       cp_vrel[i] = cp_row(i) * static_cast<int>(a.vs[2]) + cp_voff(i);
     }
+    // the next tile to copy, and the tiles that lie wholly inside the sequence
+    const uint16_t* kg = kbase + seq_start * a.ks[2];
+    const uint16_t* vg = vbase + seq_start * a.vs[2];
+    const int64_t kg_step = kBlockN * a.ks[2], vg_step = kBlockN * a.vs[2];
+    const int n_full = (seq_end - seq_start) / kBlockN;
     auto copy_tile = [&](int t, int buf) {
-      const int ks0 = seq_start + t * kBlockN;
-      const uint16_t* kg = kbase + ks0 * a.ks[2];
-      const uint16_t* vg = vbase + ks0 * a.vs[2];
-      const int last = seq_end - 1 - ks0;  // rows past the end re-read the last row: finite data the mask discards
-      const bool full = last >= kBlockN - 1;
+      const bool full = t < n_full;
 #pragma unroll
       for (int i = 0; i < C::kLoads; ++i) {
         int krel = cp_krel[i], vrel = cp_vrel[i];
-        if (!full) {
-          const int r = min(cp_row(i), last);
+        if (!full) {  // rows past the end re-read the last row: finite data the mask discards
+          const int r = min(cp_row(i), (seq_end - seq_start) - t * kBlockN - 1);
           krel = r * static_cast<int>(a.ks[2]) + cp_koff(i);
           vrel = r * static_cast<int>(a.vs[2]) + cp_voff(i);
         }
@@ -544,6 +530,23 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
                      :: "v"(static_cast<uint32_t>(krel) * 2u), "s"(kg), "s"(kl) : "memory", "m0");
         asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
                      :: "v"(static_cast<uint32_t>(vrel) * 2u), "s"(vg), "s"(vl) : "memory", "m0");
+      }
+      kg += kg_step;
+      vg += vg_step;
+    };
+    // causal / end-of-sequence mask, on the tiles from the first that needs it: the
+    // wavefront's 32 keys from kb0 on reach past its first query or the sequence's end
+    const int kb_first = seq_start + kh * 32;
+    const int t_mask = (min(qw0 - 31, seq_end - 32) - kb_first) / kBlockN +
+                       (min(qw0 - 31, seq_end - 32) >= kb_first ? 1 : 0);
+    auto mask = [&](int t, f32x16_t& s) {
+      if (t >= t_mask) {
+        const int kb0 = kb_first + t * kBlockN;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = kb0 + (r >> 3) * 16 + half * 8 + (r & 7);
+          if (key > qpos || key >= seq_end) s[r] = -__builtin_inff();
+        }
       }
     };
 
@@ -574,9 +577,14 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
     // softmax of a tile, first half: pieces 1 .. 6
     auto head = [&](int k, const f32x16_t& s) {
       if (k == 1) {
-        mx = -__builtin_inff();
+        float mh = fmaxf(s[8], s[9]);  // two chains
+        mx = fmaxf(s[0], s[1]);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+        for (int r = 2; r < 8; ++r) {
+          mx = fmaxf(mx, s[r]);
+          mh = fmaxf(mh, s[8 + r]);
+        }
+        mx = fmaxf(mx, mh);
       } else if (k == 2) {
         mx = half_max(mx) * c;
         grow = mx > m_run + 8.0f;
@@ -626,7 +634,7 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
     for (int kk = 0; kk < kSteps; ++kk) sA[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk], qf[kk], sA[0], 0, 0, 0);
 #pragma unroll
     for (int kk = 0; kk < kSteps; ++kk) read_k(1, kk);
-    mask(0, sA);
+    mask(0, sA[0]);
 #pragma unroll
     for (int k = 1; k < 8; ++k) head(k, sA[0]);
 
@@ -667,7 +675,7 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
         wait_copies(issued);
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the V operands have arrived
         __syncthreads();
-        mask(t + 1, sn);
+        mask(t + 1, sn[0]);
       }
       // ---- phase B
       __builtin_amdgcn_sched_barrier(0);
