@@ -492,7 +492,8 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
     // 63 VALU instructions and 17 exps, about 520, against 16 x 32), so half of
     // it belongs to each MFMA phase: with all of it under the scores, the two
     // wavefronts of a SIMD, which pass the barrier together, left the matrix
-    // core idle half of that phase and the VALU idle during P·V (@GQA@).
+    // core idle half of that phase and the VALU idle during P·V (B=1,
+    // T=2048, 16/4 x 128 gated: 40.4 -> 36.5 us; 8/8 heads: 36.0 -> 32.1).
     // Every operand is read a phase before its MFMA.
     //
     // LDS: a step copies tile t+3 into the stage tile t-1 left: its V operands
