@@ -83,7 +83,8 @@ struct GdArgs {
   uint16_t* w;       // [Hv, nc, plane 3, wv 4, st 4, lane 64, 8] bf16: w_x[16wv + c16][32st + 8g4 + e],
                      // w split exactly into hi + mid + lo planes
   float* u;          // [Hv, nc, js 8, wv 4, lane 64, r 4]: u[16wv + 4g4 + r][16js + c16]
-  float* aq;         // [Hv, nc, rt 4, st 2, lane 64, 8]: A[16rt + c16][32st + 8g4 + e]
+  uint16_t* aq;      // [Hv, nc, kAqChunk] bf16: planes hi, mid, lo (an exact split) of A[16rt + c16][32st + 8g4 + e],
+                     // e = 0..7 at aq_offset(rt, st, lane) of each plane
   int hk, hv, nc, nseq;
   int varlen, seq_len, nct;  // packed requests (table) or a padded batch of nct chunks per sequence
   int beta_f32, l2norm;
@@ -115,6 +116,18 @@ __device__ __forceinline__ void split3x4(const float* x, uint2& hi, uint2& mid, 
   hi = make_uint2(h01, h23);
   mid = make_uint2(m01, m23);
   lo = make_uint2(l01, l23);
+}
+
+// eight fp32 values -> three planes of eight bf16 (16 bytes per plane)
+__device__ __forceinline__ void split3x8(f32x4_t v0, f32x4_t v1, uint4& hi, uint4& mid, uint4& lo) {
+  const float va[4] = {v0[0], v0[1], v0[2], v0[3]};
+  const float vb[4] = {v1[0], v1[1], v1[2], v1[3]};
+  uint2 ha, ma, la, hb, mb, lb;
+  split3x4(va, ha, ma, la);
+  split3x4(vb, hb, mb, lb);
+  hi = make_uint4(ha.x, ha.y, hb.x, hb.y);
+  mid = make_uint4(ma.x, ma.y, mb.x, mb.y);
+  lo = make_uint4(la.x, la.y, lb.x, lb.y);
 }
 
 __device__ __forceinline__ void unpack8(uint4 raw, float* x) {
@@ -263,17 +276,26 @@ __device__ __forceinline__ void request_chunks(const GdArgs& a, int s, int* firs
 constexpr int kRowK = kD + 8;    // bf16 row stride of the row-major q/k/v tiles (272 B)
 constexpr int kRowF = kC + 4;    // fp32 row stride of the 64x64 tiles (272 B)
 constexpr int kPrepK = 0;                                   // bf16 [64][kRowK]
-constexpr int kPrepQ = kPrepK + kC * kRowK * 2;             // bf16 [64][kRowK]
+constexpr int kPrepQ = kPrepK + kC * kRowK * 2;             // bf16 [64][kRowK]; then A, fp32 [64][kRowF]
 constexpr int kPrepV = kPrepQ + kC * kRowK * 2;             // bf16 [64][kRowK]
 constexpr int kPrepL = kPrepV + kC * kRowK * 2;             // fp32 [64][kRowF]
 constexpr int kPrepG = kPrepL + kC * kRowF * 4;             // fp32 [64]  gc
 constexpr int kPrepB = kPrepG + kC * 4;                     // fp32 [64]  beta
 constexpr int kPrepBG = kPrepB + kC * 4;                    // fp32 [64]  beta e^gc
 constexpr int kPrepBytes = kPrepBG + kC * 4;
+static_assert(kC * kRowF * 4 <= kC * kRowK * 2, "A takes the place of the q tile");
 
-// position of A[i][j] in the state pass's output-wavefront operand order
-__device__ __forceinline__ int aq_index(int i, int j) {
-  return (((i >> 4) * 2 + (j >> 5)) * 64 + 16 * ((j & 31) >> 3) + (i & 15)) * 8 + (j & 7);
+// A's planes in the state pass's output-wavefront operand order: five slots of 64
+// lanes x 8 elements and one lane's zeros.  A is lower triangular: rows 0..31 have no
+// tile st = 1, and the upper lanes (8g4 >= 16) of tiles (0,0) and (2,1) are zero, so
+// the two share slot 0 and their upper lanes read the zeros.  (1,0) (2,0) (3,0) and
+// (3,1) take the slots 1..4.
+constexpr int kAqPlane = 5 * 64 * 8 + 64;  // elements per plane (a multiple of 128 bytes)
+constexpr int kAqChunk = kC * kC * 2;      // elements per chunk
+static_assert(3 * kAqPlane <= kAqChunk, "the planes of A fit in the space of the fp32 matrix");
+__device__ __forceinline__ int aq_offset(int rt, int st, int lane) {
+  if (rt == 2 * st) return (lane < 32 ? st * 32 + lane : 5 * 64) * 8;
+  return ((st == 0 ? rt : 4) * 64 + lane) * 8;
 }
 
 // Inside a 16-row block the solve reads row m of the transposed L tile in 4-wide
@@ -384,13 +406,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   }
   __syncthreads();
 
-  // Gram (k.k) and q.k lower 32x32 tiles on bf16 MFMA; wave 3 zeroes A's upper tile
-  float* gaq = a.aq + hc * kC * kC;
+  // Gram (k.k) and q.k lower 32x32 tiles on bf16 MFMA (waves 0-2)
+  float* sA = reinterpret_cast<float*>(smem + kPrepQ);
+  const int I = wv == 0 ? 0 : 1;
+  const int J = wv == 2 ? 1 : 0;
+  f32x16_t accG = {};
+  f32x16_t accA = {};
   if (wv < 3) {
-    const int I = wv == 0 ? 0 : 1;
-    const int J = wv == 2 ? 1 : 0;
-    f32x16_t accG = {};
-    f32x16_t accA = {};
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const int kc = 16 * s + 8 * (l >> 5);
@@ -400,6 +422,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
       accG = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ak, bk, accG, 0, 0, 0);
       accA = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aq, bk, accA, 0, 0, 0);
     }
+  }
+  __syncthreads();  // the q tile is free: A takes its place
+  if (wv < 3) {
     const int j = 32 * J + (l & 31);
     const float gj = sG[j];
     // gc and beta of the lane's 16 rows 32I + 8q + 4(l/32) + e, read before any is
@@ -417,13 +442,25 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
       const float e = expf(gi[r >> 2][r & 3] - gj);
       const float dec = i >= j ? e : 0.0f;
       sL[j * kRowF + i] = i > j ? (bi[r >> 2][r & 3] * accG[r]) * dec : 0.0f;  // transposed: sL[j][i] = L[i][j]
-      gaq[aq_index(i, j)] = i >= j ? (a.scale * accA[r]) * dec : 0.0f;
+      sA[i * kRowF + j] = i >= j ? (a.scale * accA[r]) * dec : 0.0f;
     }
-  } else {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) gaq[aq_index(r * 2 + (l >> 5), 32 + (l & 31))] = 0.0f;
   }
   __syncthreads();
+  // A's planes in operand order, row block wv: through LDS a lane stores 16 bytes
+  // per plane (straight from the accumulators it would be 2)
+  {
+    for (int st = 0; st <= (wv >> 1); ++st) {
+      uint16_t* ga = a.aq + hc * kAqChunk + aq_offset(wv, st, l);  // upper lanes of a shared tile store the zeros
+      const float* src_a = sA + (16 * wv + c16) * kRowF + 32 * st + 8 * g4;
+      const f32x4_t v0 = *reinterpret_cast<const f32x4_t*>(src_a);
+      const f32x4_t v1 = *reinterpret_cast<const f32x4_t*>(src_a + 4);
+      uint4 hi, mid, lo;
+      split3x8(v0, v1, hi, mid, lo);
+      *reinterpret_cast<uint4*>(ga) = hi;
+      *reinterpret_cast<uint4*>(ga + kAqPlane) = mid;
+      *reinterpret_cast<uint4*>(ga + 2 * kAqPlane) = lo;
+    }
+  }
 
   // forward substitution (I + L) x = rhs, one column per thread (wave wv owns the 64
   // columns of its lanes), in four blocks of 16 rows:
@@ -505,14 +542,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         const float* src_row = wl + (l & 15) * 64 + 32 * ch + 8 * (l >> 4);
         const f32x4_t v0 = *reinterpret_cast<const f32x4_t*>(src_row);
         const f32x4_t v1 = *reinterpret_cast<const f32x4_t*>(src_row + 4);
-        const float va[4] = {v0[0], v0[1], v0[2], v0[3]};
-        const float vb[4] = {v1[0], v1[1], v1[2], v1[3]};
-        uint2 ha, ma, la, hb, mb, lb;
-        split3x4(va, ha, ma, la);
-        split3x4(vb, hb, mb, lb);
-        *reinterpret_cast<uint4*>(gw + q * 8) = make_uint4(ha.x, ha.y, hb.x, hb.y);
-        *reinterpret_cast<uint4*>(gw + kC * kD + q * 8) = make_uint4(ma.x, ma.y, mb.x, mb.y);
-        *reinterpret_cast<uint4*>(gw + 2 * kC * kD + q * 8) = make_uint4(la.x, la.y, lb.x, lb.y);
+        uint4 hi, mid, lo;
+        split3x8(v0, v1, hi, mid, lo);
+        *reinterpret_cast<uint4*>(gw + q * 8) = hi;
+        *reinterpret_cast<uint4*>(gw + kC * kD + q * 8) = mid;
+        *reinterpret_cast<uint4*>(gw + 2 * kC * kD + q * 8) = lo;
       }
     } else {
       // u piece (rows 16b + 4(lane/16) .. +3, column 16g + lane%16) in fp32;
@@ -598,6 +632,7 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t sS[3][kSlice * kRowSB];   // state planes [col][dk]
   __shared__ __attribute__((aligned(16))) uint16_t sVd[3][kSlice * kRowVB];  // e^{gl - gc} v' planes [col][t]
   __shared__ __attribute__((aligned(16))) uint16_t sVp[3][kSlice * kRowVB];  // v' planes [col][t]
+  __shared__ __attribute__((aligned(16))) float sE[2][3 * kC];               // a chunk's exponentials (GdArgs::gc)
 
   const int tid = threadIdx.x;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -623,42 +658,49 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
     struct ChunkRegs {
       uint4 w[3][4];  // plane x, step s: w_x[16wv + c16][32s + 8g4 .. +7]      (A of w S)
       uint4 k[2][2];  // tile m, step s: k^T[32wv + 16m + c16][32s + 8g4 .. +7]  (A of k^T v')
-      float u[4];     // u[16wv + 4g4 + r][col]                                 (C layout)
-      f32x4_t dec;    // e^{gl - gc_t}, t = 16wv + 4g4 .. +3
-      float egl;      // e^{gl}
+      f32x4_t u;      // u[16wv + 4g4 + r][col]                                 (C layout)
     };
-    // Part `part` of the operand loads of chunk c: parts 0-2 are the w planes,
-    // part 3 k^T, u and the exponentials; -1 loads all of them.
-    auto load_chunk = [&](ChunkRegs& R, int c, int part = -1) {
-      c = min(c, last - 1);
-      const size_t hc = static_cast<size_t>(h) * a.nc + c;
-      const uint16_t* w = a.w + hc * 3 * kC * kD + (wv * 4 * 64 + l) * 8;
-#pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        if (part >= 0 && part != x) continue;
-#pragma unroll
-        for (int st = 0; st < 4; ++st) R.w[x][st] = *reinterpret_cast<const uint4*>(w + x * kC * kD + st * 64 * 8);
+    // The chunk to load next: uniform pointers that advance by a chunk, and stay on
+    // the request's last one.  (Addresses formed from the chunk index cost each part
+    // of the loads several 64-bit scalar multiplies, in line with the chain.)
+    const size_t hc0 = static_cast<size_t>(h) * a.nc + first;
+    const uint16_t* pw = a.w + hc0 * 3 * kC * kD;
+    const uint16_t* pk = a.kn + hc0 * kC * kD;
+    const float* pu = a.u + hc0 * kC * kD;
+    int at = first;
+    const int lane_op = (wv * 4 * 64 + l) * 8, lane_u = ((js * 4 + wv) * 64 + l) * 4;
+    // Its 17 operand loads: 4 x + st plane x of w, 12 + 2 m + st k^T, then u.
+    constexpr int kOps = 17;
+    auto load_op = [&](ChunkRegs& R, int i) {
+      if (i < 12) {
+        R.w[i >> 2][i & 3] = *reinterpret_cast<const uint4*>(pw + (i >> 2) * kC * kD + lane_op + (i & 3) * 64 * 8);
+      } else if (i < 16) {
+        R.k[(i >> 1) & 1][i & 1] = *reinterpret_cast<const uint4*>(pk + lane_op + (i & 3) * 64 * 8);
+      } else {
+        R.u = *reinterpret_cast<const f32x4_t*>(pu + lane_u);
       }
-      if (part >= 0 && part != 3) return;
-      const uint16_t* kt = a.kn + hc * kC * kD + (wv * 4 * 64 + l) * 8;
+    };
+    auto next_chunk = [&]() {
+      if (at + 1 < last) {
+        ++at;
+        pw += 3 * kC * kD;
+        pk += kC * kD;
+        pu += kC * kD;
+      }
+    };
+    auto load_ops = [&](ChunkRegs& R, int i0, int i1) {
 #pragma unroll
-      for (int m = 0; m < 2; ++m)
-#pragma unroll
-        for (int st = 0; st < 2; ++st) R.k[m][st] = *reinterpret_cast<const uint4*>(kt + (m * 2 + st) * 64 * 8);
-      const f32x4_t u4 = *reinterpret_cast<const f32x4_t*>(a.u + hc * kC * kD + ((js * 4 + wv) * 64 + l) * 4);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) R.u[r] = u4[r];
-      const float* gx = a.gc + hc * 3 * kC;
-      R.dec = *reinterpret_cast<const f32x4_t*>(gx + kC + 16 * wv + 4 * g4);
-      R.egl = gx[2 * kC];
+      for (int i = i0; i < i1; ++i) load_op(R, i);
     };
 
-    // One chunk.  The loads of chunk cp (two ahead) into P go out in four parts,
-    // each where the wavefront waits anyway (before a barrier, behind an issued
-    // MFMA group): the address unit takes about 16 cycles per 1 KiB load per CU,
-    // and one burst of all 19 would stall the in-order wavefront for most of a
-    // step.  sched_barrier keeps each part in place.
-    auto step = [&](const ChunkRegs& R, int c, ChunkRegs& P, int cp) {
+    // One chunk.  The loads of the chunk two ahead into P are spread over the step:
+    // before the barriers, where the wavefront waits anyway, and one behind each
+    // group of MFMAs.  The CU returns at most 64 B per cycle to all eight wavefronts
+    // (the data return unit is busy 75 % of the pass), so a load issued with others
+    // waits about 100 cycles in line; behind MFMAs that wait is theirs.
+    // sched_barrier keeps each in place.
+    int par = 0;  // the chunk's buffer of exponentials
+    auto step = [&](const ChunkRegs& R, ChunkRegs& P) {
       // state at the chunk start: bf16 planes to LDS (B of w S and of the output's q S)
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
@@ -670,7 +712,7 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
         *reinterpret_cast<uint2*>(sS[2] + c16 * kRowSB + dk) = pl;
       }
       __builtin_amdgcn_sched_barrier(0);
-      load_chunk(P, cp, 0);
+      load_ops(P, 0, 4);
       __builtin_amdgcn_sched_barrier(0);
       __syncthreads();
 
@@ -689,16 +731,18 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
         acc1 = mfma_bf16(R.w[0][st], sl, acc1);
         acc0 = mfma_bf16(R.w[1][st], sm, acc0);
         acc1 = mfma_bf16(R.w[2][st], sh, acc1);
+        load_op(P, 4 + st);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
-      load_chunk(P, cp, 1);
-      __builtin_amdgcn_sched_barrier(0);
+      const f32x4_t dec = *reinterpret_cast<const f32x4_t*>(sE[par] + kC + 16 * wv + 4 * g4);
+      const float egl = sE[par][2 * kC];
+      par ^= 1;
       f32x4_t vnew;
       float vdec[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         vnew[r] = R.u[r] - (acc0[r] + acc1[r]);
-        vdec[r] = vnew[r] * R.dec[r];
+        vdec[r] = vnew[r] * dec[r];
       }
       {
         const int off = c16 * kRowVB + 16 * wv + 4 * g4;
@@ -715,13 +759,13 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
         *reinterpret_cast<uint2*>(sVp[2] + off) = pl;
       }
       __builtin_amdgcn_sched_barrier(0);
-      load_chunk(P, cp, 2);
+      load_ops(P, 8, 12);
       __builtin_amdgcn_sched_barrier(0);
       __syncthreads();
 
       // S <- e^{gl} S + k^T (e^{gl - gc} v'), dk rows 32wv..32wv+31
-      f32x4_t st0 = {S[0][0] * R.egl, S[0][1] * R.egl, S[0][2] * R.egl, S[0][3] * R.egl};
-      f32x4_t st1 = {S[1][0] * R.egl, S[1][1] * R.egl, S[1][2] * R.egl, S[1][3] * R.egl};
+      f32x4_t st0 = {S[0][0] * egl, S[0][1] * egl, S[0][2] * egl, S[0][3] * egl};
+      f32x4_t st1 = {S[1][0] * egl, S[1][1] * egl, S[1][2] * egl, S[1][3] * egl};
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
         const int off = c16 * kRowVB + 32 * st + 8 * g4;
@@ -730,14 +774,18 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
         const uint4 dl = *reinterpret_cast<const uint4*>(sVd[2] + off);
         st0 = mfma_bf16(R.k[0][st], dh, st0);
         st1 = mfma_bf16(R.k[1][st], dh, st1);
+        load_op(P, 12 + 2 * st);
+        __builtin_amdgcn_sched_barrier(0);
         st0 = mfma_bf16(R.k[0][st], dm, st0);
         st1 = mfma_bf16(R.k[1][st], dm, st1);
+        load_op(P, 13 + 2 * st);
+        __builtin_amdgcn_sched_barrier(0);
         st0 = mfma_bf16(R.k[0][st], dl, st0);
         st1 = mfma_bf16(R.k[1][st], dl, st1);
+        if (st == 1) load_op(P, 16);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
-      load_chunk(P, cp, 3);
-      __builtin_amdgcn_sched_barrier(0);
+      next_chunk();
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         S[0][r] = st0[r];
@@ -749,12 +797,14 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
 
     if (first < last) {
       ChunkRegs A, B, Cr;
-      load_chunk(A, first);
-      load_chunk(B, first + 1);
+      load_ops(A, 0, kOps);
+      next_chunk();
+      load_ops(B, 0, kOps);
+      next_chunk();
       for (int c = first; c < last; c += 3) {
-        step(A, c, Cr, c + 2);
-        if (c + 1 < last) step(B, c + 1, A, c + 3);
-        if (c + 2 < last) step(Cr, c + 2, B, c + 4);
+        step(A, Cr);
+        if (c + 1 < last) step(B, A);
+        if (c + 2 < last) step(Cr, B);
       }
     }
 
@@ -775,92 +825,132 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
     const size_t o_row = static_cast<size_t>(a.hv) * kD;
     struct OutRegs {
       uint4 q[4];       // q[16rt + c16][32st + 8g4 .. +7]
-      f32x4_t av[2][2];  // A[16rt + c16][32st + 8g4 + 4i .. +3]
-      f32x4_t eg;       // e^{gc_t}, t = 16rt + 4g4 .. +3
+      uint4 a[2][3];    // plane x of A[16rt + c16][32st + 8g4 .. +7]; st = 1 for rt >= 2 only
+      f32x4_t e;        // wavefront rt = 0: the chunk's exponentials 4l .. 4l + 3, for every wavefront
     };
-    auto load_out = [&](OutRegs& R, int c) {
-      c = min(c, last - 1);
-      const size_t hc = static_cast<size_t>(h) * a.nc + c;
-      const uint16_t* qp = a.qn + hc * kC * kD + (rt * 4 * 64 + l) * 8;
-#pragma unroll
-      for (int st = 0; st < 4; ++st) R.q[st] = *reinterpret_cast<const uint4*>(qp + st * 64 * 8);
-      const float* ap = a.aq + hc * kC * kC + (rt * 2 * 64 + l) * 8;
-#pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        R.av[st][0] = *reinterpret_cast<const f32x4_t*>(ap + st * 64 * 8);
-        R.av[st][1] = *reinterpret_cast<const f32x4_t*>(ap + st * 64 * 8 + 4);
+    // the chunk to load next, as the chain's
+    const size_t hc0 = static_cast<size_t>(h) * a.nc + first;
+    const uint16_t* pq = a.qn + hc0 * kC * kD;
+    const uint16_t* pa = a.aq + hc0 * kAqChunk;
+    const float* pg = a.gc + hc0 * 3 * kC;
+    int at = first;
+    const int lane_q = (rt * 4 * 64 + l) * 8, lane_e = 4 * min(l, 3 * kC / 4 - 1);
+    const int lane_a[2] = {aq_offset(rt, 0, l), aq_offset(rt, 1, l)};
+    // its 11 loads: 0 .. 3 q, 4 .. 9 the A planes, 10 the exponentials
+    auto load_op = [&](OutRegs& R, int i) {
+      if (i < 4) {
+        R.q[i] = *reinterpret_cast<const uint4*>(pq + lane_q + i * 64 * 8);
+      } else if (i < 10) {
+        if (i < 7 || rt >= 2)
+          R.a[(i - 4) / 3][(i - 4) % 3] = *reinterpret_cast<const uint4*>(pa + lane_a[(i - 4) / 3] + (i - 4) % 3 * kAqPlane);
+      } else if (rt == 0) {
+        R.e = *reinterpret_cast<const f32x4_t*>(pg + lane_e);
       }
-      R.eg = *reinterpret_cast<const f32x4_t*>(a.gc + hc * 3 * kC + 16 * rt + 4 * g4);
     };
-    auto split8v = [](f32x4_t v0, f32x4_t v1, uint4& hi, uint4& mid, uint4& lo) {
-      const float va[4] = {v0[0], v0[1], v0[2], v0[3]};
-      const float vb[4] = {v1[0], v1[1], v1[2], v1[3]};
-      uint2 ha, ma, la, hb, mb, lb;
-      split3x4(va, ha, ma, la);
-      split3x4(vb, hb, mb, lb);
-      hi = make_uint4(ha.x, ha.y, hb.x, hb.y);
-      mid = make_uint4(ma.x, ma.y, mb.x, mb.y);
-      lo = make_uint4(la.x, la.y, lb.x, lb.y);
+    auto next_chunk = [&]() {
+      if (at + 1 < last) {
+        ++at;
+        pq += kC * kD;
+        pa += kAqChunk;
+        pg += 3 * kC;
+      }
     };
-    // the barriers match the chain's step: the first finds the chunk-start
-    // state planes in sS, the second the v' planes in sVp
-    auto out_step = [&](const OutRegs& R, int c, OutRegs& P, int cp) {
+    auto load_out = [&](OutRegs& R) {
+#pragma unroll
+      for (int i = 0; i < 11; ++i) load_op(R, i);
+      next_chunk();
+    };
+    // the request's rows: chunk c of it holds rows [row, min(row + 64, row_end)), row
+    // advancing with c
+    int row = 0, row_end = 0;
+    if (first < last) {
+      int tail_row, tail_len;
+      chunk_rows(a, first, &row, &tail_len);
+      chunk_rows(a, last - 1, &tail_row, &tail_len);
+      row_end = tail_row + tail_len;
+    }
+    uint16_t* po = a.o + static_cast<size_t>(row) * o_row + h * kD;  // uniform: the lane's part is lane_o
+    const int lane_row = 16 * rt + 4 * g4 + 2 * (l & 1);  // of the two rows this lane stores
+    const int lane_o = lane_row * a.hv * kD + (col & ~1);
+    // The barriers match the chain's step: the first finds the chunk-start
+    // state planes in sS, the second the v' planes in sVp.  The chain waits here
+    // for these wavefronts as much as they for it, so what they need not do is not
+    // done: A comes split from prep, the zero half of its upper rows is skipped, a
+    // chunk's rows follow from the last's, every LDS read of a phase is issued before
+    // its MFMAs (a dependent chain) and one load of the chunk two ahead behind each
+    // of those (B=1, T=2048: state pass 46.8 -> 42 us, prep 24.6 -> 25.4; 64 requests
+    // of 64 tokens: 164 -> 148 us for the call).
+    int par = 0;  // the chunk's buffer of exponentials
+    auto out_step = [&](const OutRegs& R, const OutRegs& N, OutRegs& P) {
       __syncthreads();
-      // the chain's operand reads of the state planes go first: the A split and
-      // the next chunk's loads (no LDS) come before this wavefront's own reads
-      uint4 ah[2], am[2], al[2];
-      split8v(R.av[0][0], R.av[0][1], ah[0], am[0], al[0]);
-      load_out(P, cp);
-      __builtin_amdgcn_sched_barrier(0);
       f32x4_t acc1 = {};
+      uint4 sp[4][3];
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int x = 0; x < 3; ++x) sp[st][x] = *reinterpret_cast<const uint4*>(sS[x] + c16 * kRowSB + 32 * st + 8 * g4);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
-        const int off = c16 * kRowSB + 32 * st + 8 * g4;
-        const uint4 sh = *reinterpret_cast<const uint4*>(sS[0] + off);
-        const uint4 sm = *reinterpret_cast<const uint4*>(sS[1] + off);
-        const uint4 sl = *reinterpret_cast<const uint4*>(sS[2] + off);
-        acc1 = mfma_bf16(R.q[st], sh, acc1);
-        acc1 = mfma_bf16(R.q[st], sm, acc1);
-        acc1 = mfma_bf16(R.q[st], sl, acc1);
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+          acc1 = mfma_bf16(R.q[st], sp[st][x], acc1);
+          if (st * 3 + x < 11) load_op(P, st * 3 + x);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
+      next_chunk();
       __syncthreads();
-      // likewise the chain's reads of the e^{gl - gc} v' planes go first
-      split8v(R.av[1][0], R.av[1][1], ah[1], am[1], al[1]);
-      __builtin_amdgcn_sched_barrier(0);
       f32x4_t acc2 = {};
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
+        if (st == 1 && rt < 2) break;  // A is lower triangular: zero right of column 31 in rows 0..31
         const int off = c16 * kRowVB + 32 * st + 8 * g4;
         const uint4 b0 = *reinterpret_cast<const uint4*>(sVp[0] + off);
         const uint4 b1 = *reinterpret_cast<const uint4*>(sVp[1] + off);
         const uint4 b2 = *reinterpret_cast<const uint4*>(sVp[2] + off);
-        acc2 = mfma_bf16(ah[st], b0, acc2);
-        acc2 = mfma_bf16(ah[st], b1, acc2);
-        acc2 = mfma_bf16(am[st], b0, acc2);
-        acc2 = mfma_bf16(ah[st], b2, acc2);
-        acc2 = mfma_bf16(am[st], b1, acc2);
-        acc2 = mfma_bf16(al[st], b0, acc2);
+        acc2 = mfma_bf16(R.a[st][0], b0, acc2);
+        acc2 = mfma_bf16(R.a[st][0], b1, acc2);
+        acc2 = mfma_bf16(R.a[st][1], b0, acc2);
+        acc2 = mfma_bf16(R.a[st][0], b2, acc2);
+        acc2 = mfma_bf16(R.a[st][1], b1, acc2);
+        acc2 = mfma_bf16(R.a[st][2], b0, acc2);
       }
-      int r0, L;
-      chunk_rows(a, c, &r0, &L);
+      const f32x4_t eg = *reinterpret_cast<const f32x4_t*>(sE[par] + 16 * rt + 4 * g4);
+      par ^= 1;
+      if (rt == 0) *reinterpret_cast<f32x4_t*>(sE[par] + lane_e) = N.e;  // read after the next step's first barrier
+      float val[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * rt + 4 * g4 + r;
-        if (t < L) {
-          const float val = (a.scale * R.eg[r]) * acc1[r] + acc2[r];
-          a.o[static_cast<size_t>(r0 + t) * o_row + h * kD + col] = static_cast<uint16_t>(fd_pack2(val, 0.0f));
-        }
+      for (int r = 0; r < 4; ++r) val[r] = (a.scale * eg[r]) * acc1[r] + acc2[r];
+      // lanes 2i and 2i + 1 (columns c, c + 1) swap two of their four rows, so that each
+      // stores two rows of a column pair
+      const uint32_t p01 = fd_pack2(val[0], val[1]), p23 = fd_pack2(val[2], val[3]);
+      const bool odd = l & 1;
+      const uint32_t own = odd ? p23 : p01;
+      const uint32_t other = static_cast<uint32_t>(
+          __builtin_amdgcn_mov_dpp(static_cast<int>(odd ? p01 : p23), 0xB1, 0xF, 0xF, false));  // quad_perm [1,0,3,2]
+      const uint32_t c0 = odd ? other : own, c1 = odd ? own : other;
+      const uint32_t lo = (c0 & 0xffffu) | (c1 << 16), hi = (c0 >> 16) | (c1 & 0xffff0000u);
+      if (row + kC <= row_end) {  // uniform: every row of the chunk is valid
+        *reinterpret_cast<uint32_t*>(po + lane_o) = lo;
+        *reinterpret_cast<uint32_t*>(po + lane_o + a.hv * kD) = hi;
+      } else {
+        if (row + lane_row < row_end) *reinterpret_cast<uint32_t*>(po + lane_o) = lo;
+        if (row + lane_row + 1 < row_end) *reinterpret_cast<uint32_t*>(po + lane_o + a.hv * kD) = hi;
       }
+      row += kC;
+      po += kC * o_row;
     };
 
     if (first < last) {
       OutRegs A, B, Cr;
-      load_out(A, first);
-      load_out(B, first + 1);
+      load_out(A);
+      load_out(B);
+      if (rt == 0) *reinterpret_cast<f32x4_t*>(sE[0] + lane_e) = A.e;
       for (int c = first; c < last; c += 3) {
-        out_step(A, c, Cr, c + 2);
-        if (c + 1 < last) out_step(B, c + 1, A, c + 3);
-        if (c + 2 < last) out_step(Cr, c + 2, B, c + 4);
+        out_step(A, B, Cr);
+        if (c + 1 < last) out_step(B, Cr, A);
+        if (c + 2 < last) out_step(Cr, A, B);
       }
     }
   }
@@ -897,7 +987,7 @@ GdLayout gd_layout(int64_t nc, int64_t hv, int64_t nseq, int64_t tokens) {
   L.u = off;
   off = al(off + hc * kC * kD * 4);
   L.aq = off;
-  off = al(off + hc * kC * kC * 4);
+  off = al(off + hc * kAqChunk * 2);
   L.ob = off;
   off = al(off + static_cast<size_t>(tokens) * hv * kD * 2);
   L.total = off;
@@ -999,7 +1089,7 @@ int gd_run(const void* q, const void* k, const void* v, const float* g, const vo
   a.kn = reinterpret_cast<uint16_t*>(ws + lay.kn);
   a.w = reinterpret_cast<uint16_t*>(ws + lay.w);
   a.u = reinterpret_cast<float*>(ws + lay.u);
-  a.aq = reinterpret_cast<float*>(ws + lay.aq);
+  a.aq = reinterpret_cast<uint16_t*>(ws + lay.aq);
   a.hk = k_heads;
   a.hv = v_heads;
   a.nc = static_cast<int>(nc);
