@@ -615,6 +615,8 @@ constexpr int kRowVB = kC + 8;   // bf16 row stride of a transposed v' plane (14
 
 constexpr int kStateThreads = 512;
 
+// PREFETCH: the output wavefronts fetch the operands into L2 ahead of the loads.
+template <bool PREFETCH>
 __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
   // Block b runs on XCD b % 8.  The 8 column slices of one head (which read the
   // same w / k / q / A tiles) go to one XCD and share its L2; the heads of one
@@ -860,6 +862,39 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
       for (int i = 0; i < 11; ++i) load_op(R, i);
       next_chunk();
     };
+    // L2 prefetch: the operands of the chunk four ahead, one 4-byte load
+    // of each 128-byte line; the 32 output wavefronts of a head's slices take a share
+    // each, and a lane keeps one line's address.
+    const char* pf_line = nullptr;
+    int pf_step = 0, pf_left = 0;  // chunks from pf_line's to the request's last
+    if constexpr (PREFETCH) {
+      constexpr int kRegions = 6;
+      constexpr int kBytes[kRegions] = {3 * kC * kD * 2, kC * kD * 2, kC * kD * 4, kC * kD * 2, 3 * kAqPlane * 2, 3 * kC * 4};
+      constexpr int kStep[kRegions] = {3 * kC * kD * 2, kC * kD * 2, kC * kD * 4, kC * kD * 2, kAqChunk * 2, 3 * kC * 4};
+      constexpr int kLines = (kBytes[0] + kBytes[1] + kBytes[2] + kBytes[3] + kBytes[4] + kBytes[5]) / 128;
+      constexpr int kShare = (kLines + 4 * kSlices - 1) / (4 * kSlices);
+      static_assert(kShare <= 64, "one line per lane");
+      const void* const base[kRegions] = {a.w, a.kn, a.u, a.qn, a.aq, a.gc};
+      const int line = l < kShare ? (js * 4 + rt) * kShare + l : kLines;
+      int begin = 0;
+#pragma unroll
+      for (int r = 0; r < kRegions; ++r) {
+        if (line >= begin && line < begin + kBytes[r] / 128) {
+          pf_line = static_cast<const char*>(base[r]) + hc0 * kStep[r] + (line - begin) * 128;
+          pf_step = kStep[r];
+          pf_left = last - 1 - first;
+        }
+        begin += kBytes[r] / 128;
+      }
+    }
+    auto prefetch = [&]() {
+      int v = 0;
+      if (pf_left >= 0 && pf_line != nullptr) v = *reinterpret_cast<const int*>(pf_line);
+      pf_line += pf_step;
+      --pf_left;
+      return v;
+    };
+    int pf_value = 0;
     // the request's rows: chunk c of it holds rows [row, min(row + 64, row_end)), row
     // advancing with c
     int row = 0, row_end = 0;
@@ -900,6 +935,10 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
         }
       }
       next_chunk();
+      if constexpr (PREFETCH) {
+        asm volatile("" ::"v"(pf_value));  // the last step's line, long arrived
+        pf_value = prefetch();
+      }
       __syncthreads();
       f32x4_t acc2 = {};
 #pragma unroll
@@ -946,6 +985,13 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
       OutRegs A, B, Cr;
       load_out(A);
       load_out(B);
+      if constexpr (PREFETCH) {  // the loads above are chunks 0 and 1, the steps fetch chunk 4 on
+        pf_line += 2 * pf_step;
+        pf_left -= 2;
+        const int v2 = prefetch();
+        pf_value = prefetch();
+        asm volatile("" ::"v"(v2));
+      }
       if (rt == 0) *reinterpret_cast<f32x4_t*>(sE[0] + lane_e) = A.e;
       for (int c = first; c < last; c += 3) {
         out_step(A, B, Cr);
@@ -1111,7 +1157,17 @@ int gd_run(const void* q, const void* k, const void* v, const float* g, const vo
       hipLaunchKernelGGL(gd_prep_kernel<false>, dim3(static_cast<unsigned>(nc * v_heads)), dim3(kThreads), 0, s, a);
   }
   const int64_t units = (nseq * v_heads + 7) / 8 * 8;  // (request, head) units, rounded up to the XCDs
-  hipLaunchKernelGGL(gd_state_kernel, dim3(static_cast<unsigned>(units * kSlices)), dim3(kStateThreads), 0, s, a);
+  // Intermediates that do not fit the 256 MB memory-side cache beside q, k, v and the
+  // output come from HBM, too late for loads two chunks ahead: long chains then fetch
+  // four chunks ahead into L2 (B=1, 16 heads: T=8192, 270 MB, 339 -> 282 us; T=7000,
+  // 232 MB, 248 -> 230; T=6000, 198 MB, 191.9 -> 188.8; T=4096, 135 MB, 123.6 ->
+  // 129.1; B=4, T=2048 236 -> 217).  Short chains pay for it (40 requests of 10 to
+  // 200 tokens: 164 -> 177 us).
+  const dim3 state_grid(static_cast<unsigned>(units * kSlices));
+  if (lay.ob > 208LL << 20 && nc >= 24 * nseq)
+    hipLaunchKernelGGL(gd_state_kernel<true>, state_grid, dim3(kStateThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL(gd_state_kernel<false>, state_grid, dim3(kStateThreads), 0, s, a);
   const int rc = fd_check_launch("fd_gated_delta_fwd");
   if (rc != FD_OK || norm == nullptr || total == 0) return rc;
   // the layer's gated RMSNorm over the raw output rows (one row per token and value head)

@@ -268,3 +268,27 @@ def test_packed_requests_equal_the_same_requests_alone(hk, hv, lengths):
         alone, state = rule(*(t[:, a:b].contiguous() for t in (q, k, v, g, beta)), use_qk_l2norm_in_kernel=True,
                             output_final_state=True)
         assert torch.equal(out[:, a:b], alone) and torch.equal(final[i], state[0]), (i, a, b)
+
+
+@pytest.mark.parametrize("B,T,packed", [(2, 4096, False), (1, 7001, True)])
+def test_chains_that_prefetch_equal_those_that_do_not(B, T, packed):
+    """Above 208 MiB of intermediates the state pass fetches ahead into L2; the rows and states equal those of the
+    same sequences alone or with fewer heads, which do not."""
+    announce(f"gated delta prefetch B={B} T={T} packed={packed}")
+    q, k, v, g, beta = (t.cuda() for t in _inputs(T, 16, 16, 91, B=B))
+    rule = _rule()
+    kw = dict(use_qk_l2norm_in_kernel=True, output_final_state=True)
+    if packed:
+        cu = [0, 70, T]
+        kw["cu_seqlens"] = torch.tensor(cu, dtype=torch.int32, device="cuda")
+        from fastdecisions_amd.gated_delta_kernel import workspace_bytes
+        assert workspace_bytes(1, T, 16, 2) - T * 16 * 128 * 2 > 208 << 20
+    out, final = rule(q, k, v, g, beta, **kw)
+    if packed:
+        half = [t[:, :, :8].contiguous() for t in (q, k, v, g, beta)]
+        few, states = rule(*half, **kw)
+        assert torch.equal(out[:, :, :8], few) and torch.equal(final[:, :8], states)
+    else:
+        for b in range(B):
+            alone, state = rule(*(t[b:b + 1].contiguous() for t in (q, k, v, g, beta)), **kw)
+            assert torch.equal(out[b], alone[0]) and torch.equal(final[b], state[0])
