@@ -13,6 +13,7 @@ export every symbol listed in ``SIGNATURES``.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from pathlib import Path
@@ -183,8 +184,11 @@ def check(name: str, code: int) -> None:
         raise KernelError(name, code, lib().fd_last_error().decode(errors="replace"))
 
 
+_I64x4 = ctypes.c_int64 * 4
+
+
 def strides4(t) -> ctypes.Array:
-    return (ctypes.c_int64 * 4)(*t.stride())
+    return _I64x4(*t.stride())
 
 
 def ptr(t) -> int | None:
@@ -192,4 +196,14 @@ def ptr(t) -> int | None:
 
 
 def stream_handle(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The device's current stream as a raw handle (the value of ``current_stream(device).cuda_stream``
+    without building the stream object: 0.1 us instead of 2)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device(device):
+    """``torch.cuda.device(device)``, or nothing to enter where it is the current device already."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)

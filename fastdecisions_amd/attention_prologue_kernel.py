@@ -50,7 +50,7 @@ def attention_prologue(q: torch.Tensor, k: torch.Tensor, q_weight: torch.Tensor,
         for t in (cos, sin):
             if t.dtype != torch.bfloat16 or t.device != q.device or not t.is_contiguous() or t.data_ptr() % 16:
                 raise ValueError("cos and sin must be contiguous, 16-byte aligned BF16 on q's device")
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         q_out = torch.empty((B, T, Hq, D), device=q.device, dtype=torch.bfloat16)
         k_out = torch.empty((B, T, Hkv, D), device=q.device, dtype=torch.bfloat16)
         _lib.check("fd_attn_prologue_fwd", _lib.lib().fd_attn_prologue_fwd(

@@ -103,7 +103,7 @@ def chunk_gated_delta_rule(
     if norm is not None:
         z, norm_weight, norm_eps = norm
         norm_args = _norm_args(z, norm_weight, B, T, Hv, Dv, value.device)
-    with torch.cuda.device(value.device):
+    with _lib.on_device(value.device):
         out = torch.empty((B, T, Hv, Dv), device=value.device, dtype=torch.bfloat16)
         final = torch.empty(state_shape, device=value.device, dtype=torch.float32) if output_final_state else None
         nbytes = workspace_bytes(B, T, Hv, n_seqs)

@@ -43,7 +43,7 @@ def gated_rms_norm(x: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, ep
     if weight.shape != (D,) or weight.dtype not in _W_DTYPES or weight.device != x.device or not weight.is_contiguous():
         raise ValueError(f"weight must be a contiguous BF16 or FP32 vector [{D}] on x's device")
     rows = x.numel() // D
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         out = torch.empty_like(x)
         _lib.check("fd_gated_rmsnorm_fwd", _lib.lib().fd_gated_rmsnorm_fwd(
             x.data_ptr(), gate.data_ptr(), ts, hs, heads, weight.data_ptr(), _W_DTYPES[weight.dtype],
@@ -58,7 +58,7 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
         raise ValueError("gate_up must be contiguous and 16-byte aligned")
     width = gate_up.shape[-1] // 2
     rows = gate_up.numel() // gate_up.shape[-1]
-    with torch.cuda.device(gate_up.device):
+    with _lib.on_device(gate_up.device):
         out = torch.empty((*gate_up.shape[:-1], width), device=gate_up.device, dtype=torch.bfloat16)
         _lib.check("fd_silu_mul_fwd", _lib.lib().fd_silu_mul_fwd(
             gate_up.data_ptr(), gate_up.shape[-1], out.data_ptr(), rows, width, _lib.stream_handle(gate_up.device)))
@@ -78,7 +78,7 @@ def silu_mul_split(gate_up1: torch.Tensor, gate_up2: torch.Tensor) -> torch.Tens
         raise ValueError("gate_up1 and gate_up2 must have the same leading shape and device")
     w1, w2 = gate_up1.shape[-1] // 2, gate_up2.shape[-1] // 2
     rows = gate_up1.numel() // gate_up1.shape[-1]
-    with torch.cuda.device(gate_up1.device):
+    with _lib.on_device(gate_up1.device):
         out = torch.empty((*gate_up1.shape[:-1], w1 + w2), device=gate_up1.device, dtype=torch.bfloat16)
         _lib.check("fd_silu_mul_split_fwd", _lib.lib().fd_silu_mul_split_fwd(
             gate_up1.data_ptr(), gate_up1.shape[-1], w1, gate_up2.data_ptr(), gate_up2.shape[-1], w2, out.data_ptr(),

@@ -24,7 +24,7 @@ def hbm_copy(src: torch.Tensor, dst: torch.Tensor, chunks_per_thread: int = 1, b
     nbytes = src.numel() * src.element_size()
     if dst.numel() * dst.element_size() != nbytes:
         raise ValueError("src and dst must hold the same number of bytes")
-    with torch.cuda.device(src.device):
+    with _lib.on_device(src.device):
         _lib.check("fd_hbm_copy", _lib.lib().fd_hbm_copy(src.data_ptr(), dst.data_ptr(), nbytes, chunks_per_thread,
                                                          block, _lib.stream_handle(src.device)))
     return dst

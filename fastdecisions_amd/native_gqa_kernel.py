@@ -64,15 +64,17 @@ def native_gqa_attention(
             raise ValueError("Q, K and V must share a CUDA device")
         if tensor.dtype != torch.bfloat16:
             raise ValueError("Q, K and V must be BF16")
-        if tensor.stride(-1) != 1:
+        sb, sh, st, sd = tensor.stride()
+        if sd != 1:
             raise ValueError("The feature dimension must be contiguous")
-        if tensor.data_ptr() % 16 or any(s % 8 for s in tensor.stride()[:3]):
+        if tensor.data_ptr() % 16 or (sb | sh | st) % 8:
             raise ValueError("Q, K and V rows must be 16-byte aligned")
 
     if gate is not None:
         if gate.shape != q.shape or gate.dtype != torch.bfloat16 or gate.device != q.device:
             raise ValueError("gate must be a BF16 tensor shaped like Q on Q's device")
-        if gate.stride(-1) != 1 or gate.data_ptr() % 16 or any(s % 8 for s in gate.stride()[:3]):
+        sb, sh, st, sd = gate.stride()
+        if sd != 1 or gate.data_ptr() % 16 or (sb | sh | st) % 8:
             raise ValueError("gate rows must be contiguous and 16-byte aligned")
 
     n_seqs = 0
@@ -95,16 +97,16 @@ def native_gqa_attention(
     if scale is None:
         scale = head_dim ** -0.5
 
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         # Physical layout [B, T, Hq, D], logical layout [B, Hq, T, D] (ref: :145-151).
         output = torch.empty(
             (batch, seq_len, q_heads, head_dim), device=q.device, dtype=q.dtype
         ).permute(0, 2, 1, 3)
         lib = _lib.lib()
-        # workspace of the key split of long query tiles (head_dim 256 with few work items;
-        # 0 bytes: the kernel runs unsplit)
+        # workspace of the key split of long query tiles (padded head_dim-256 batches with few
+        # work items; 0 bytes: the kernel runs unsplit)
         nbytes = 0
-        if key_split:
+        if key_split and head_dim == 256 and cu_ptr is None:
             nbytes = lib.fd_gqa_workspace_bytes(batch, q_heads, kv_heads, seq_len, head_dim, n_seqs,
                                                 int(max_seqlen))
             if nbytes < 0:

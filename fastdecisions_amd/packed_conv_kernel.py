@@ -67,8 +67,7 @@ def _check_conv(input_qkv, weight, bias, key_dim, value_dim, head_k_dim, head_v_
             raise ValueError(f"bias must be a contiguous BF16 vector [{C}] on input_qkv's device")
     if activation not in _ACTIVATIONS:
         raise ValueError("activation must be 'silu' or None")
-    tensors = [input_qkv, weight] + ([bias] if bias is not None else [])
-    if any(t.data_ptr() % 16 for t in tensors):
+    if input_qkv.data_ptr() % 16 or weight.data_ptr() % 16 or (bias is not None and bias.data_ptr() % 16):
         raise ValueError("Inputs must be aligned to 16 bytes")
 
     n_seqs = 0
@@ -87,7 +86,10 @@ def _check_conv(input_qkv, weight, bias, key_dim, value_dim, head_k_dim, head_v_
 def _alloc_qkv(input_qkv, B, T, key_dim, value_dim, head_k_dim, head_v_dim):
     q = torch.empty((B, T, key_dim // head_k_dim, head_k_dim), device=input_qkv.device, dtype=input_qkv.dtype)
     k = torch.empty_like(q)
-    v = torch.empty((B, T, value_dim // head_v_dim, head_v_dim), device=input_qkv.device, dtype=input_qkv.dtype)
+    if (value_dim, head_v_dim) == (key_dim, head_k_dim):
+        v = torch.empty_like(q)
+    else:
+        v = torch.empty((B, T, value_dim // head_v_dim, head_v_dim), device=input_qkv.device, dtype=input_qkv.dtype)
     return q, k, v
 
 
@@ -105,7 +107,7 @@ def prep_qkv(
 ):
     B, T, key_dim, value_dim, row_stride, width, cu_ptr, n_seqs = _check_conv(
         input_qkv, weight, bias, key_dim, value_dim, head_k_dim, head_v_dim, activation, cu_seqlens)
-    with torch.cuda.device(input_qkv.device):
+    with _lib.on_device(input_qkv.device):
         q, k, v = _alloc_qkv(input_qkv, B, T, key_dim, value_dim, head_k_dim, head_v_dim)
         lib = _lib.lib()
         _lib.check("fd_packed_conv_strided_fwd", lib.fd_packed_conv_strided_fwd(
@@ -140,7 +142,7 @@ def prep_qkv_gates(
     gB, gT, hidden, H = _check_gate_projection(hidden_states, gate_weight, a_log, dt_bias)
     if (gB, gT) != (B, T) or hidden_states.device != input_qkv.device:
         raise ValueError("hidden_states must be [B, T, hidden] with input_qkv's B and T, on its device")
-    with torch.cuda.device(input_qkv.device):
+    with _lib.on_device(input_qkv.device):
         q, k, v = _alloc_qkv(input_qkv, B, T, key_dim, value_dim, head_k_dim, head_v_dim)
         decay = torch.empty((B, T, H), device=input_qkv.device, dtype=torch.float32)
         beta = torch.empty((B, T, H), device=input_qkv.device, dtype=torch.bfloat16)

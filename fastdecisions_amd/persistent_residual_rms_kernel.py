@@ -65,7 +65,7 @@ def fused_add_rms_norm(
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """Return ``(rmsnorm(residual + x), residual + x)`` (both bf16, fresh tensors)."""
     width = _validate(x, residual, weight)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         out = torch.empty_like(x)
         new_residual = torch.empty_like(x)
         _launch(x, residual, weight, out, new_residual, width, eps, gain_offset)
@@ -75,7 +75,7 @@ def fused_add_rms_norm(
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, *, gain_offset: bool = True) -> torch.Tensor:
     """RMSNorm of ``x`` over its last dimension (Qwen3.5 ``(1 + w)`` gain by default)."""
     width = _validate(x, None, weight)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         out = torch.empty_like(x)
         _launch(x, None, weight, out, None, width, eps, gain_offset)
     return out
@@ -96,7 +96,7 @@ def residual_rms(a: torch.Tensor, b: torch.Tensor, weight: torch.Tensor, eps: fl
     if not all(t.is_contiguous() for t in (a, b, weight)):
         raise ValueError("All inputs must be contiguous")
     width = _validate(b, a, weight)
-    with torch.cuda.device(a.device):
+    with _lib.on_device(a.device):
         out = torch.empty(a.shape, device=a.device, dtype=torch.bfloat16)
         _launch(b, a, weight, out, None, width, eps, True)
     return out

@@ -45,7 +45,7 @@ def slot_readout(hidden: torch.Tensor, norm_weight: torch.Tensor, letters: torch
     pos = _index(slot_positions, N, hidden.device, "slot_positions")
     nop = None if nopts is None else _index(nopts, N, hidden.device, "nopts")
     K = letters.shape[0]
-    with torch.cuda.device(hidden.device):
+    with _lib.on_device(hidden.device):
         logits = torch.empty((N, K), device=hidden.device, dtype=torch.float32)
         probs = torch.empty((N, K), device=hidden.device, dtype=torch.float32) if with_probs else None
         _lib.check("fd_slot_readout_fwd", _lib.lib().fd_slot_readout_fwd(

@@ -50,7 +50,7 @@ def gate_transform(a: torch.Tensor, b: torch.Tensor, a_log: torch.Tensor, dt_bia
         if t.stride(2) != 1 or t.stride(0) != T * t.stride(1):
             raise ValueError("a and b must be row-contiguous views [B, T, H] (unit head stride, packed rows)")
     _check_params(a_log, dt_bias, H, a.device)
-    with torch.cuda.device(a.device):
+    with _lib.on_device(a.device):
         decay = torch.empty((B, T, H), device=a.device, dtype=torch.float32)
         beta = torch.empty((B, T, H), device=a.device, dtype=torch.bfloat16)
         _lib.check("fd_gate_transform_fwd", _lib.lib().fd_gate_transform_fwd(
@@ -97,7 +97,7 @@ def gate_projection(x: torch.Tensor, weight: torch.Tensor, a_log: torch.Tensor, 
     if ab is not None and (ab.shape != (B, T, 2 * H) or ab.dtype != torch.bfloat16 or not ab.is_contiguous()
                            or ab.device != x.device):
         raise ValueError("ab must be a contiguous BF16 [B, T, 2H] tensor on x's device")
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         decay = torch.empty((B, T, H), device=x.device, dtype=torch.float32)
         beta = torch.empty((B, T, H), device=x.device, dtype=torch.bfloat16)
         _lib.check("fd_gate_proj_fwd", _lib.lib().fd_gate_proj_fwd(

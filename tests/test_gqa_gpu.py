@@ -334,3 +334,16 @@ def test_key_split_equals_the_unsplit_kernel(Hq, Hkv, T, D, gated, oracle):
     assert (diff <= ulp).all()
     if not gated:
         assert (split - sdpa_fp32(q, k, v)).abs().max().item() <= ATOL
+
+
+def test_launches_follow_the_current_stream_and_device():
+    """The raw handle is the current stream's, also inside a stream context, and the device guard enters
+    nothing on the current device."""
+    from fastdecisions_amd import _lib
+    dev = torch.device("cuda", torch.cuda.current_device())
+    assert _lib.stream_handle(dev) == torch.cuda.current_stream(dev).cuda_stream
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert _lib.stream_handle(dev) == side.cuda_stream
+    with _lib.on_device(dev):
+        assert torch.cuda.current_device() == dev.index
