@@ -15,11 +15,10 @@
 //   the other issues MFMAs.  head_dim 256 runs 4 wavefronts (register budget).
 // * K and V tiles (64 keys) are copied global -> LDS with global_load_lds
 //   (no staging registers, no VALU), one barrier per tile.  For head_dim
-//   <= 128 the ring has 4 stages and the loop is software-pipelined: while a
-//   wavefront finishes tile t (mask, softmax, P·V), the scores of tile t+1
-//   are computed, one MFMA of that dependent chain after each of eight pieces
-//   of the softmax, so the VALU work issues while the MFMAs run; tiles t+2 and
-//   t+3 are in flight.
+//   <= 128 the ring has 4 stages and the loop is software-pipelined in two
+//   phases: the scores of tile t+1 run with the second half of tile t's
+//   softmax between their MFMAs, then the P·V of tile t with the first half of
+//   tile t+1's softmax between them; tiles t+2 and t+3 are in flight.
 // * head_dim 256: one wavefront per head (4 per workgroup), each walking
 //   32-key blocks; the P·V of block j-1 and the scores of block j+1 are
 //   issued with the softmax of block j between their MFMAs, over 2-stage K
@@ -116,7 +115,7 @@ struct Cfg {
   static constexpr int kLoads = kBlockN * kChunksRow / kThreads;  // global_load_lds per thread per K (or V) tile
   static constexpr int kStageBytes = 2 * kTileBytes;         // K tile + V tile
   // Pipelined loop (two wavefronts per (head, query block) and 4 stages in
-  // LDS): the scores of tile t+1 are computed while tile t is finished, and
+  // LDS): tile t+1's scores and tile t's P·V each carry half of a softmax, and
   // tiles t+2, t+3 are in flight.  head_dim 256 (one wavefront per (head,
   // query block)) has 2 stages, used as separate K and V rings.
   static constexpr bool kPipe = KSPLIT > 1 && 4 * kStageBytes <= 160 * 1024;
