@@ -234,6 +234,15 @@ __device__ __forceinline__ void store_rows(const f32x16_t (&o)[D / 32], float in
   }
 }
 
+// Copies 16 bytes per lane from `base` (uniform) + `off` to 1 KiB of LDS at
+// `lds`, in flight until a vmcnt wait: an asm that the compiler does not count.
+// The hardware needs one wait state between a write of M0 and the copy that
+// reads it; the compiler keeps it for its own copies, not inside an asm.
+__device__ __forceinline__ void copy_to_lds(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+
 // Rows [start, end) of packed request s, clamped to [0, T], so a malformed
 // offset table cannot move an access outside q/k/v/o.
 __device__ __forceinline__ void packed_bounds(const GqaArgs& a, int s, int* start, int* end) {
@@ -546,10 +555,8 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
         }
         const uint32_t kl = lds0 + static_cast<uint32_t>(buf * C::kTileBytes + (i * C::kWaves + wave) * 1024);
         const uint32_t vl = kl + static_cast<uint32_t>(C::kStages * C::kTileBytes);
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                     :: "v"(static_cast<uint32_t>(krel) * 2u), "s"(kg), "s"(kl) : "memory", "m0");
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                     :: "v"(static_cast<uint32_t>(vrel) * 2u), "s"(vg), "s"(vl) : "memory", "m0");
+        copy_to_lds(kg, static_cast<uint32_t>(krel) * 2u, kl);
+        copy_to_lds(vg, static_cast<uint32_t>(vrel) * 2u, vl);
       }
       kg += kg_step;
       vg += vg_step;
@@ -769,8 +776,7 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
         const int r = min(4 * kRowsPer * i + crow, last);
         const int rel = r * stride + (is_v ? cv_off : ck_off[i % kKPer]);
         const uint32_t lds = stage_base + static_cast<uint32_t>((i * C::kWaves + wave) * 1024);
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                     :: "v"(static_cast<uint32_t>(rel) * 2u), "s"(g), "s"(lds) : "memory", "m0");
+        copy_to_lds(g, static_cast<uint32_t>(rel) * 2u, lds);
       }
     };
     // K operand (block bl of a tile, step kk): row bl*32 + sigma(col), logical chunk 2kk + half;
