@@ -432,19 +432,17 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
   // Q^T as MFMA B operand: lane supplies Q[qpos][16kk + 8*half + 0..7].
   // The loops issue their copies as asm and count them themselves; the compiler,
   // which does not see them, must not be left with loads of its own to wait for.
-  // So Q is read with asm too, before any copy, and the prologue's copy wait
-  // covers it.  Rows past the end read the last row and are zeroed after that wait.
+  // So Q is loaded before any copy, and the prologue waits for it and the copies
+  // its first scores read (vmcnt 0) before it issues the others.  (Q loads in asm,
+  // counted with the copies, left registers in flight that the compiler took as
+  // written; this form measured equal at 64/128 and 72.8 -> 73.2 us at 2x2048 of
+  // 8/2 heads of 256.)  Rows past the end read the last row, zeroed after the wait.
   bf16x8_t qf[D / 16];
   {
-    typedef unsigned u32x4q_t __attribute__((ext_vector_type(4)));
     const int qrow = qvalid ? qpos : seq_end - 1;
     const uint16_t* qp = qbase + qrow * a.qs[2] + half * 8;
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
-      u32x4q_t raw;
-      asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(raw) : "v"(qp), "i"(kk * 32) : "memory");
-      qf[kk] = __builtin_bit_cast(bf16x8_t, raw);
-    }
+    for (int kk = 0; kk < D / 16; ++kk) qf[kk] = *reinterpret_cast<const bf16x8_t*>(qp + kk * 16);
   }
   auto q_arrived = [&]() {
 #pragma unroll
@@ -647,12 +645,12 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
         __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(0));
     };
 
-    // Prologue: tiles 0..2 in flight, tiles 0 and 1 landed; scores of tile 0 and the head of its softmax.
+    // Prologue: Q and tiles 0 and 1 landed, tile 2 in flight; scores of tile 0 and the head of its softmax.
     copy_tile(0, 0);
     if (ntiles > 1) copy_tile(1, 1);
+    wait_copies(false);
+    q_arrived();
     if (ntiles > 2) copy_tile(2, 2);
-    wait_copies(ntiles > 2);
-    q_arrived();  // the Q loads are older than every copy
     __syncthreads();
 #pragma unroll
     for (int kk = 0; kk < kSteps; ++kk) read_k(0, kk);
@@ -746,7 +744,8 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
     // the VALU work runs under the MFMAs.  K and V have 2-stage rings of whole
     // tiles: K(u) is copied in step 2u-3 and read in steps 2u-1, 2u; V(u) is
     // copied in step 2u-1 and read in steps 2u+1, 2u+2.  Copies and LDS
-    // operand reads are asm with explicit waits (see the Q loads).
+    // operand reads are asm with explicit waits: the compiler counts neither, so
+    // it must not have loads of its own in flight (see the Q loads).
     constexpr int kKk = D / 16;   // score MFMAs per block (and P·V MFMAs)
     constexpr int kNdb = D / 32;  // O^T blocks
     constexpr int RB = CR * 16;   // bytes per K / V row in LDS
@@ -812,13 +811,12 @@ __global__ __launch_bounds__(256 * KSPLIT, 1) void gqa_fwd_kernel(GqaArgs a) {
       }
     };
 
-    // prologue: K0, K1, V0 in flight; scores of block 0 once K0 has landed
+    // prologue: Q and K0 landed, K1 and V0 in flight; scores of block 0
     copy_tile(0, false);
+    __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(0));
+    q_arrived();
     if (ntiles > 1) copy_tile(1, false);
     copy_tile(0, true);
-    if (ntiles > 1) __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(2 * C::kLoads));
-    else __builtin_amdgcn_s_waitcnt(C::waitcnt_vm(C::kLoads));
-    q_arrived();  // the Q loads are older than every copy
     __syncthreads();
     f32x16_t S[2];   // scores of block b in S[b & 1]
     bf16x8_t P[2][2];  // P of block b in P[b & 1] (two 16-key slices)

@@ -40,3 +40,35 @@ def test_a_wait_state_between_m0_and_the_copy_that_reads_it(kernels):
                 copies += 1
                 assert before[1][:1] != ["m0"], f"{name}: {before[3]} directly before {now[3]}"
     assert copies
+
+
+def _registers(operand):
+    kind, span = operand[0], operand[1:].strip("[]").split(":")
+    return {(kind, r) for r in range(int(span[0]), int(span[-1]) + 1)} if span[0].isdigit() else set()
+
+
+def test_no_asm_leaves_a_global_load_into_registers_in_flight(kernels):
+    """The compiler takes an asm's outputs as written: a global load there either goes to LDS or is waited for there."""
+    for name, ins in kernels.items():
+        for i, (op, _, in_asm, text) in enumerate(ins):
+            if in_asm and op.startswith(("global_load_dword", "buffer_load_dword")):
+                rest = ins[i + 1:]
+                end = next(j for j, step in enumerate(rest) if not step[2])
+                assert any(step[0] == "s_waitcnt" and "vmcnt(0)" in step[3] for step in rest[:end]), f"{name}: {text}"
+
+
+def test_registers_of_asm_lds_reads_are_untouched_until_their_wait(kernels):
+    """In program order, no instruction names a register that an LDS read issued by an asm may still write."""
+    for name, ins in kernels.items():
+        flight = []  # LDS instructions not waited for: (registers an asm read writes, text)
+        for op, operands, in_asm, text in ins:
+            if op == "s_waitcnt":
+                count = re.search(r"lgkmcnt\((\d+)\)", text)
+                if count:
+                    flight = flight[max(0, len(flight) - int(count[1])):] if int(count[1]) else []
+                continue
+            named = set().union(*map(_registers, operands)) if operands else set()
+            hit = next((read for regs, read in flight if regs & named), None)
+            assert hit is None, f"{name}: {text} while {hit} is in flight"
+            if op.startswith("ds_"):
+                flight.append((_registers(operands[0]) if in_asm and op.startswith("ds_read") else set(), text))
