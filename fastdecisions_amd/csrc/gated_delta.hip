@@ -73,7 +73,7 @@ struct GdArgs {
   int32_t* len;      // [nc]  valid rows of each chunk (0 = unused)
   int32_t* first;    // [N+1] first chunk of each request
   int32_t* order;    // [N]   requests, longest first
-  float* gc;         // [Hv, nc, 3, 64]: e^{gc_t}, e^{gl - gc_t}, then e^{gl} (gl = gc of the last row)
+  float* gc;         // [Hv, nc, 3, 64]: e^{gc_t}, e^{gl - gc_t}, then e^{gl} 64 times (gl = gc of the last row)
   // q and A are stored in the state pass's output-wavefront operand order
   // (lane = 16 * g4 + c16): every load there reads 1-2 KiB contiguous
   uint16_t* qn;      // [Hv, nc, rt 4, st 4, lane 64, 8] bf16: q[16rt + c16][32st + 8g4 + e]
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     float* gx = a.gc + hc * 3 * kC;
     gx[l] = eg;
     gx[kC + l] = expf(gl - gv);
-    if (l == 0) gx[2 * kC] = expf(gl);
+    gx[2 * kC + l] = expf(gl);  // in every place: the state pass copies the block whole
   }
 #pragma unroll
   for (int it = 0; it < 4; ++it) {

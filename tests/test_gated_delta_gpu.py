@@ -292,3 +292,33 @@ def test_chains_that_prefetch_equal_those_that_do_not(B, T, packed):
         for b in range(B):
             alone, state = rule(*(t[b:b + 1].contiguous() for t in (q, k, v, g, beta)), **kw)
             assert torch.equal(out[b], alone[0]) and torch.equal(final[b], state[0])
+
+
+@pytest.mark.parametrize("B,T,hk,hv,cu", [(1, 130, 2, 2, None), (2, 64, 1, 2, None), (1, 200, 1, 1, [0, 1, 1, 66, 200])])
+def test_a_call_writes_the_workspace_it_reads(B, T, hk, hv, cu):
+    """The state pass reads every chunk's exponentials, q, k^T, w and u whole: over a workspace of all-one bits (a NaN in
+    either type) none of those words is left, whatever the chunk's length."""
+    from fastdecisions_amd import _lib
+    announce(f"gated delta workspace written B={B} T={T} hv={hv} cu={cu}")
+    q, k, v, g, beta = (t.cuda() for t in _inputs(T, hk, hv, 5, B=B))
+    n = 0 if cu is None else len(cu) - 1
+    table = None if cu is None else torch.tensor(cu, dtype=torch.int32, device="cuda")
+    nc, nseq = (B * -(-T // 64), B) if cu is None else (-(-T // 64) + n, n)
+    used = nc if cu is None else sum(-(-(b - a) // 64) for a, b in zip(cu[:-1], cu[1:]))
+    nbytes = _lib.lib().fd_gated_delta_workspace_bytes(B, T, hv, 128, 128, n)
+    work = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")
+    out = torch.empty((B, T, hv, 128), dtype=torch.bfloat16, device="cuda")
+    _lib.check("fd_gated_delta_fwd", _lib.lib().fd_gated_delta_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(), out.data_ptr(), None, None,
+        work.data_ptr(), nbytes, B, T, hk, hv, 128, 128, 128 ** -0.5, _lib.FD_DTYPE_BF16, 1, _lib.ptr(table), n,
+        _lib.stream_handle(q.device)))
+    at = 0
+    for size in (4 * nc, 4 * nc, 4 * (nseq + 1), 4 * nseq):  # the chunk table
+        at = -(-(at + size) // 256) * 256
+    for name, per in (("exponentials", 3 * 64 * 4), ("q", 64 * 128 * 2), ("k^T", 64 * 128 * 2), ("w", 3 * 64 * 128 * 2),
+                      ("u", 64 * 128 * 4)):
+        block = work[at:at + hv * nc * per].view(torch.int32).view(hv, nc, per // 4)
+        left = int((block[:, :used] == -1).sum())
+        assert left == 0, f"{name}: {left} words of {used} chunks not written"
+        assert bool((block[:, used:] == -1).all()), name  # the layout above is the kernel's
+        at = -(-(at + hv * nc * per) // 256) * 256
