@@ -72,7 +72,6 @@ struct GdArgs {
   int32_t* row0;     // [nc]  first packed row of each chunk
   int32_t* len;      // [nc]  valid rows of each chunk (0 = unused)
   int32_t* first;    // [N+1] first chunk of each request
-  int32_t* order;    // [N]   requests, longest first
   float* gc;         // [Hv, nc, 3, 64]: e^{gc_t}, e^{gl - gc_t}, then e^{gl} 64 times (gl = gc of the last row)
   // q and A are stored in the state pass's output-wavefront operand order
   // (lane = 16 * g4 + c16): every load there reads 1-2 KiB contiguous
@@ -84,7 +83,7 @@ struct GdArgs {
                      // w split exactly into hi + mid + lo planes
   float* u;          // [Hv, nc, js 8, wv 4, lane 64, r 4]: u[16wv + 4g4 + r][16js + c16]
   uint16_t* aq;      // [Hv, nc, kAqChunk] bf16: planes hi, mid, lo (an exact split) of A[16rt + c16][32st + 8g4 + e],
-                     // e = 0..7 at aq_offset(rt, st, lane) of each plane
+                     // e = 0..7 at aq_offset(rt, st, lane) of each plane; behind them order_entry
   int hk, hv, nc, nseq;
   int varlen, seq_len, nct;  // packed requests (table) or a padded batch of nct chunks per sequence
   int beta_f32, l2norm;
@@ -172,10 +171,22 @@ __device__ __forceinline__ uint4 l2norm_row8(uint4 raw) {
 // request by a scan of their chunk counts, then every chunk's request by a
 // binary search, one chunk per thread (a thread per request that walked the
 // request's chunks took 12.8 us for requests of up to 8002 tokens; this takes 4.6).
-// `order` lists the requests longest first, so that the state pass starts the
+// order_entry lists the requests longest first, so that the state pass starts the
 // longest chains first (by counting, up to kTableThreads requests; more keep
 // their own order: their chains are many and short).
 constexpr int kTableThreads = 1024;
+
+// A's three planes in a chunk of GdArgs::aq (see aq_offset)
+constexpr int kAqPlane = 5 * 64 * 8 + 64;  // elements per plane (a multiple of 128 bytes)
+constexpr int kAqChunk = kC * kC * 2;      // elements per chunk
+static_assert(3 * kAqPlane + 2 <= kAqChunk, "the planes of A and an entry of `order` fit in the space of the fp32 matrix");
+// Entry `i` of the requests' order, longest first (packed requests): behind A's planes
+// in chunk i, so that the table takes no room of its own and the no-allocation
+// scratch, a fixed size, takes every call it took without it.  There are at least as
+// many chunks as requests.
+__device__ __forceinline__ int32_t* order_entry(const GdArgs& a, int i) {
+  return reinterpret_cast<int32_t*>(a.aq + static_cast<size_t>(i) * kAqChunk + 3 * kAqPlane);
+}
 
 __device__ __forceinline__ int request_rows(const int32_t* cu, int s, int total, int* start) {
   *start = min(max(cu[s], 0), total);
@@ -232,10 +243,10 @@ __global__ __launch_bounds__(kTableThreads) void gd_chunk_table(const int32_t* _
       if (s < nseq) {
         int rank = 0;
         for (int o = 0; o < nseq; ++o) rank += chunks[o] > n || (chunks[o] == n && o < s);
-        a.order[rank] = s;
+        *order_entry(a, rank) = s;
       }
     } else if (s < nseq) {
-      a.order[s] = s;
+      *order_entry(a, s) = s;
     }
     __syncthreads();
   }
@@ -290,9 +301,6 @@ static_assert(kC * kRowF * 4 <= kC * kRowK * 2, "A takes the place of the q tile
 // tile st = 1, and the upper lanes (8g4 >= 16) of tiles (0,0) and (2,1) are zero, so
 // the two share slot 0 and their upper lanes read the zeros.  (1,0) (2,0) (3,0) and
 // (3,1) take the slots 1..4.
-constexpr int kAqPlane = 5 * 64 * 8 + 64;  // elements per plane (a multiple of 128 bytes)
-constexpr int kAqChunk = kC * kC * 2;      // elements per chunk
-static_assert(3 * kAqPlane <= kAqChunk, "the planes of A fit in the space of the fp32 matrix");
 __device__ __forceinline__ int aq_offset(int rt, int st, int lane) {
   if (rt == 2 * st) return (lane < 32 ? st * 32 + lane : 5 * 64) * 8;
   return ((st == 0 ? rt : 4) * 64 + lane) * 8;
@@ -627,7 +635,7 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
   if (unit >= a.nseq * a.hv) return;
   const int js = blockIdx.x / 8 % kSlices;
   const int h = unit % a.hv;
-  const int sq = a.varlen ? a.order[unit / a.hv] : unit / a.hv;
+  const int sq = a.varlen ? *order_entry(a, unit / a.hv) : unit / a.hv;
   int first, last;
   request_chunks(a, sq, &first, &last);
 
@@ -1006,7 +1014,7 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
 // intermediates GdArgs describes, and `ob`, the raw bf16 output rows
 // [tokens, Hv, 128] that the gated norm reads (fd_gated_delta_norm_fwd only).
 struct GdLayout {
-  size_t row0, len, first, order, gc, qn, kn, w, u, aq, ob, total;
+  size_t row0, len, first, gc, qn, kn, w, u, aq, ob, total;
 };
 
 GdLayout gd_layout(int64_t nc, int64_t hv, int64_t nseq, int64_t tokens) {
@@ -1020,8 +1028,6 @@ GdLayout gd_layout(int64_t nc, int64_t hv, int64_t nseq, int64_t tokens) {
   off = al(off + static_cast<size_t>(nc) * 4);
   L.first = off;
   off = al(off + static_cast<size_t>(nseq + 1) * 4);
-  L.order = off;
-  off = al(off + static_cast<size_t>(nseq) * 4);
   L.gc = off;
   off = al(off + hc * 3 * kC * 4);
   L.qn = off;
@@ -1129,7 +1135,6 @@ int gd_run(const void* q, const void* k, const void* v, const float* g, const vo
   a.row0 = reinterpret_cast<int32_t*>(ws + lay.row0);
   a.len = reinterpret_cast<int32_t*>(ws + lay.len);
   a.first = reinterpret_cast<int32_t*>(ws + lay.first);
-  a.order = reinterpret_cast<int32_t*>(ws + lay.order);
   a.gc = reinterpret_cast<float*>(ws + lay.gc);
   a.qn = reinterpret_cast<uint16_t*>(ws + lay.qn);
   a.kn = reinterpret_cast<uint16_t*>(ws + lay.kn);

@@ -314,3 +314,32 @@ def test_gqa_key_split_only_at_head_dim_256():
         assert nbytes > 0 and nbytes % 16 == 0, (B, Hq, Hkv, T)
     assert lib.fd_gqa_workspace_bytes(1, 8, 2, 2048, 256, 4, 700) == 0  # packed requests
     assert lib.fd_gqa_workspace_bytes(4, 8, 2, 2048, 256, 0, 0) == 0  # enough work items
+
+
+def test_gated_delta_workspace_is_no_larger_than_its_fp32_layout():
+    """The fixed no-allocation scratch accepts every call whose chunk table, exponentials, q, k, w planes, u, A as an fp32
+    matrix and output rows fit it: the workspace is never larger than that layout, also where it fills the scratch exactly."""
+    from fastdecisions_amd import _lib
+    lib = _lib.lib()
+    limit = 83886080  # FD_GD_SCRATCH_BYTES
+    assert f"#define FD_GD_SCRATCH_BYTES {limit}LL" in HEADER.read_text()
+
+    def fp32_layout(batch, T, hv, n):
+        total = batch * T
+        nc, seqs = (-(-total // 64) + n, n) if n else (batch * -(-T // 64), batch)
+        sizes = [4 * nc, 4 * nc, 4 * (seqs + 1)]
+        sizes += [hv * nc * s for s in (3 * 64 * 4, 64 * 128 * 2, 64 * 128 * 2, 3 * 64 * 128 * 2, 64 * 128 * 4, 64 * 64 * 4)]
+        return sum(-(-s // 256) * 256 for s in sizes + [total * hv * 256])
+
+    def need(batch, T, hv, n):
+        return lib.fd_gated_delta_workspace_bytes(batch, T, hv, 128, 128, n)
+
+    # exactly at the limit
+    for T, n in ((36171, 0), (35656, 9), (30503, 100)):
+        assert fp32_layout(1, T, 1, n) == limit and need(1, T, 1, n) <= limit
+    for hv in (1, 2, 16, 32):
+        for T in (1, 63, 64, 65, 500, 2048, 36171):
+            for n in (0, 1, 2, 63, 64, 65, 128, 1024, 1025, 5000):
+                assert need(1, T, hv, n) <= fp32_layout(1, T, hv, n), (T, hv, n)
+            for batch in (2, 7, 64):
+                assert need(batch, T, hv, 0) <= fp32_layout(batch, T, hv, 0), (batch, T, hv)

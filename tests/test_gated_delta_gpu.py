@@ -313,7 +313,7 @@ def test_a_call_writes_the_workspace_it_reads(B, T, hk, hv, cu):
         work.data_ptr(), nbytes, B, T, hk, hv, 128, 128, 128 ** -0.5, _lib.FD_DTYPE_BF16, 1, _lib.ptr(table), n,
         _lib.stream_handle(q.device)))
     at = 0
-    for size in (4 * nc, 4 * nc, 4 * (nseq + 1), 4 * nseq):  # the chunk table
+    for size in (4 * nc, 4 * nc, 4 * (nseq + 1)):  # the chunk table
         at = -(-(at + size) // 256) * 256
     for name, per in (("exponentials", 3 * 64 * 4), ("q", 64 * 128 * 2), ("k^T", 64 * 128 * 2), ("w", 3 * 64 * 128 * 2),
                       ("u", 64 * 128 * 4)):
