@@ -79,8 +79,8 @@ struct GqaArgs {
   int hpw;        // query heads per workgroup
   int qpw;        // 32-query blocks per workgroup (hpw * qpw == 4)
   int q_heads, kv_heads, seq_len;
-  // Key split of the long query tiles (padded batches with few work items, see
-  // split_tiles): the n_split longest tiles of every (sequence, head group) run as
+  // Key split of the long query tiles (padded batches with fewer work items
+  // than CUs): the n_split longest tiles of every (sequence, head group) run as
   // two items over the two halves of their key tiles, each writing its
   // unnormalised (o, running max, denominator) to `part`; gqa_combine_kernel
   // merges them.
@@ -1121,44 +1121,22 @@ bool stride_ok(const int64_t s[4]) {
   return true;
 }
 
-// Sizes shared by the launcher and fd_gqa_workspace_bytes.
-struct GqaShape {
-  int hpw, qpw, n_qtiles, n_hgroups, n_slots;
-  int64_t items;
-};
-
-// Key split (head_dim 256 only): a padded batch with few work items for the
-// 256 CUs of the MI355X (e.g. B=1, T=2048, 8/2 heads of 256: 128 items) runs
-// the longest half of its query tiles as two items over the two halves
+// Key split (head_dim 256 only): a padded batch with fewer work items than
+// the 256 CUs of the MI355X (e.g. B=1, T=2048, 8/2 heads of 256: 128 items)
+// runs the longest half of its query tiles as two items over the two halves
 // of their key tiles, merged by gqa_combine_kernel.  The merge rounds
 // differently from the whole-tile loop, so a head_dim-256 row depends on
 // whether the split ran (the caller turns it off by passing no workspace).
 // head_dim 64 and 128 never split: at one item per CU (B=1, T=2048, 16/4
 // heads of 128) the split measured no faster, and without it every launch of
 // these head dims runs the same loop, whatever the batch.
-//
-// Fewer items than CUs always split.  From there to kSplitLongUpTo items the CUs
-// that took a long tile still end last, and halving those tiles pays only where
-// it saves more than the second launch and its traffic (about 35 MB) cost: for
-// tiles of at least kSplitLongTiles key tiles, and only where the groups share
-// the 8 XCDs evenly, as the split deals them (whole -> split us):
-//   8/2 heads, B=1: T=4096 (256 items) 143 -> 124, 5100 (320) 168 -> 149;
-//     6200 (388) 204 -> 226, 8192 (512) 295 -> 335
-//   4/1, T=8192 (256) 254 -> 187, T=10000 (313) 310 -> 250; 4/4, T=8192 (256)
-//     256 -> 190; 8/8, T=4096 (256) 138 -> 111
-//   shorter tiles: 8/2 B=4 T=1024 (256) 42 -> 54, B=2 T=2500 (316) 88 -> 91
-//   uneven groups: 12/3, T=3000 (282) 102 -> 117, T=4096 (384) 141 -> 207
 constexpr int64_t kSplitBelow = 256;
-constexpr int64_t kSplitLongUpTo = 320;
-constexpr int kSplitLongTiles = 64;
 
 // Query tiles of every (sequence, head group) that the key split halves, or 0.
-int split_tiles(const GqaShape& g, int seq_len, bool varlen, int head_dim) {
-  if (head_dim != 256 || varlen || g.n_qtiles < 4 || g.n_qtiles + g.n_qtiles / 2 > kMaxUnits) return 0;
-  const int64_t groups = static_cast<int64_t>(g.n_hgroups) * g.n_slots;
-  const bool long_tiles = g.items <= kSplitLongUpTo && seq_len > (kSplitLongTiles - 1) * kBlockN &&
-                          groups > 0 && kNumXcd % groups == 0;
-  return g.items < kSplitBelow || long_tiles ? g.n_qtiles / 2 : 0;
+int split_tiles(int n_qtiles, int64_t items, bool varlen, int head_dim) {
+  if (head_dim != 256 || varlen || items >= kSplitBelow || n_qtiles < 4 || n_qtiles + n_qtiles / 2 > kMaxUnits)
+    return 0;
+  return n_qtiles / 2;
 }
 
 // The unit table of a split launch: whole tiles and halves of the n_split
@@ -1190,6 +1168,11 @@ int64_t split_bytes(int64_t n_groups, int n_split, int head_dim) {
   return n_groups * n_split * 2 * 4 * 64 * static_cast<int64_t>(head_dim / 2 + 4) * 4;
 }
 
+// Sizes shared by the launcher and fd_gqa_workspace_bytes.
+struct GqaShape {
+  int hpw, qpw, n_qtiles, n_hgroups, n_slots;
+  int64_t items;
+};
 GqaShape gqa_shape(int batch, int q_heads, int kv_heads, int seq_len, int n_seqs, int max_seqlen, bool varlen) {
   GqaShape g;
   const int group = q_heads / kv_heads;
@@ -1269,7 +1252,7 @@ int gqa_launch(const void* q, const void* k, const void* v, void* out, const int
   FD_REQUIRE(g.items < 2147483647LL / 2, FD_ERR_INVALID_ARGUMENT, "fd_gqa_fwd: problem too large");
   const bool varlen = cu_seqlens != nullptr;
   a.n_groups = g.n_hgroups * g.n_slots;
-  a.n_split = split_tiles(g, seq_len, varlen, head_dim);
+  a.n_split = split_tiles(g.n_qtiles, g.items, varlen, head_dim);
   a.part = static_cast<float*>(workspace);
   if (a.n_split > 0 && (workspace == nullptr || !fd_aligned16(workspace) ||
                         workspace_bytes < split_bytes(a.n_groups, a.n_split, head_dim)))
@@ -1351,6 +1334,6 @@ extern "C" int64_t fd_gqa_workspace_bytes(int batch, int q_heads, int kv_heads, 
   const bool varlen = n_seqs > 0;
   if (varlen && (batch != 1 || max_seqlen < 0 || max_seqlen > seq_len)) return FD_ERR_INVALID_ARGUMENT;
   const GqaShape g = gqa_shape(batch, q_heads, kv_heads, seq_len, n_seqs, max_seqlen, varlen);
-  const int n_split = split_tiles(g, seq_len, varlen, head_dim);
+  const int n_split = split_tiles(g.n_qtiles, g.items, varlen, head_dim);
   return n_split > 0 ? split_bytes(static_cast<int64_t>(g.n_hgroups) * g.n_slots, n_split, head_dim) : 0;
 }

@@ -134,8 +134,8 @@ FD_API int fd_gqa_fwd(const void* q, const void* k, const void* v, void* out,
  *
  * Causal attention gives the query tiles near the end of a sequence up to
  * twice the average work; when a padded batch has fewer work items than the
- * GPU has CUs (B=1, T=2048, 8/2 heads of 256: 128), or hardly more and very
- * long tiles (B=1, T=4096 to 5120), those tiles set the kernel's length.  With a workspace of at least this size the longest half
+ * GPU has CUs (B=1, T=2048, 8/2 heads of 256: 128), those tiles set the
+ * kernel's length.  With a workspace of at least this size the longest half
  * of the tiles of every (sequence, head group) run as two work items over the
  * two halves of their key tiles, and a second launch on the same stream
  * merges the halves (their running maxima and denominators) and stores the

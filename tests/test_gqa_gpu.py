@@ -336,21 +336,23 @@ def test_key_split_equals_the_unsplit_kernel(Hq, Hkv, T, D, gated, oracle):
         assert (split - sdpa_fp32(q, k, v)).abs().max().item() <= ATOL
 
 
-@pytest.mark.parametrize("Hq,Hkv,T,splits", [(8, 2, 4096, True), (8, 2, 5120, True), (8, 2, 5121, False),
-                                             (8, 8, 4033, True), (4, 1, 8193, True), (12, 3, 3000, False)])
-def test_long_tiles_split_with_a_few_more_items_than_cus(Hq, Hkv, T, splits):
-    """head_dim 256, 256 to 320 work items: the key split at the edges of its rule (items, tile length,
-    groups that do not divide the XCDs), each against the whole tiles to one bf16 step."""
+@pytest.mark.parametrize("B,Hq,Hkv,T", [(1, 8, 2, 4096), (1, 8, 2, 4065), (1, 8, 2, 5120), (1, 8, 8, 4033), (1, 4, 1, 8193),
+                                        (2, 8, 2, 2048)])
+def test_head_dim_256_runs_whole_from_as_many_items_as_cus(B, Hq, Hkv, T):
+    """From 256 work items on a head_dim-256 call never splits its tiles, however long they are: it asks for no
+    workspace, and by default a request's rows are bit-identical alone (key_split off) and beside another one."""
     from fastdecisions_amd import _lib
     from fastdecisions_amd.native_gqa_kernel import native_gqa_attention
-    announce(f"gqa key split of long tiles T={T} {Hq}/{Hkv}x256")
-    assert (_lib.lib().fd_gqa_workspace_bytes(1, Hq, Hkv, T, 256, 0, 0) > 0) == splits
-    q, k, v = model_layout(1, Hq, Hkv, T, 256, 1300 + Hq, 256 ** -0.5)
-    split = native_gqa_attention(q, k, v).float()
-    whole = native_gqa_attention(q, k, v, key_split=False).float()
-    assert ((split - whole).abs() <= (whole.abs() * 2.0 ** -7).clamp_min(2.0 ** -14)).all()
-    if not splits:
-        assert torch.equal(split, whole)
+    announce(f"gqa whole tiles B={B} T={T} {Hq}/{Hkv}x256")
+    assert _lib.lib().fd_gqa_workspace_bytes(B, Hq, Hkv, T, 256, 0, 0) == 0
+    q, k, v = model_layout(B, Hq, Hkv, T, 256, 1300 + Hq, 256 ** -0.5)
+    o = native_gqa_attention(q, k, v)
+    for b in range(B):
+        one = [t[b:b + 1] for t in (q, k, v)]
+        assert torch.equal(o[b:b + 1], native_gqa_attention(*one, key_split=False))
+    padded = native_gqa_attention(*(torch.cat([t, t.flip(2)]).transpose(1, 2).contiguous().transpose(1, 2)
+                                    for t in (q, k, v)))
+    assert torch.equal(padded[:B], o)
 
 
 def test_launches_follow_the_current_stream_and_device():
