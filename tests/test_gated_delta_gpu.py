@@ -270,6 +270,15 @@ def test_packed_requests_equal_the_same_requests_alone(hk, hv, lengths):
         assert torch.equal(out[:, a:b], alone) and torch.equal(final[i], state[0]), (i, a, b)
 
 
+def _prefetches(B, T, heads, n_seqs):
+    """Whether the launcher's state pass fetches ahead: more than 208 MiB of intermediates (the workspace without the
+    output rows) and on average 24 chunks per request."""
+    from fastdecisions_amd.gated_delta_kernel import workspace_bytes
+    chunks = -(-T // 64) + n_seqs if n_seqs else B * -(-T // 64)
+    return (workspace_bytes(B, T, heads, n_seqs) - B * T * heads * 128 * 2 > 208 << 20
+            and chunks >= 24 * (n_seqs or B))
+
+
 @pytest.mark.parametrize("B,T,packed", [(2, 4096, False), (1, 7001, True)])
 def test_chains_that_prefetch_equal_those_that_do_not(B, T, packed):
     """Above 208 MiB of intermediates the state pass fetches ahead into L2; the rows and states equal those of the
@@ -279,16 +288,17 @@ def test_chains_that_prefetch_equal_those_that_do_not(B, T, packed):
     rule = _rule()
     kw = dict(use_qk_l2norm_in_kernel=True, output_final_state=True)
     if packed:
-        cu = [0, 70, T]
-        kw["cu_seqlens"] = torch.tensor(cu, dtype=torch.int32, device="cuda")
-        from fastdecisions_amd.gated_delta_kernel import workspace_bytes
-        assert workspace_bytes(1, T, 16, 2) - T * 16 * 128 * 2 > 208 << 20
+        kw["cu_seqlens"] = torch.tensor([0, 70, T], dtype=torch.int32, device="cuda")
+    n_seqs = 2 if packed else 0
+    assert _prefetches(B, T, 16, n_seqs)
     out, final = rule(q, k, v, g, beta, **kw)
     if packed:
+        assert not _prefetches(1, T, 8, n_seqs)
         half = [t[:, :, :8].contiguous() for t in (q, k, v, g, beta)]
         few, states = rule(*half, **kw)
         assert torch.equal(out[:, :, :8], few) and torch.equal(final[:, :8], states)
     else:
+        assert not _prefetches(1, T, 16, 0)
         for b in range(B):
             alone, state = rule(*(t[b:b + 1].contiguous() for t in (q, k, v, g, beta)), **kw)
             assert torch.equal(out[b], alone[0]) and torch.equal(final[b], state[0])

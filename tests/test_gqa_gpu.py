@@ -7,6 +7,8 @@ constant V); varlen equal to per-request attention.
 """
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -200,21 +202,35 @@ def test_varlen_equals_per_request():
         assert (o[:, :, a:b].float() - ref).abs().max().item() <= ATOL
 
 
-@pytest.mark.parametrize("Hq,Hkv,D,lengths", [
-    (16, 4, 128, [1]),
-    (16, 4, 128, [33, 0, 1, 2048, 32, 64, 1000]),           # equal and unequal tile counts, an empty request
-    (16, 4, 64, [(7 * i) % 91 for i in range(150)]),        # more requests than lanes
-    (12, 4, 128, [300, 129, 127, 513]),                     # 3 heads per group: 128-query tiles, 12 head groups
-    (9, 9, 64, [(31 * i) % 257 for i in range(65)]),        # 9 head groups: one more than XCDs
-    (4, 2, 64, [(13 * i) % 40 for i in range(255)] + [900]),  # the most requests that are looked up
-    (4, 2, 64, [(13 * i) % 40 for i in range(256)] + [900]),  # one more: dealt request by request
-    (4, 2, 64, [40 + (13 * i) % 40 for i in range(100)]),   # like lengths: the same
-    (8, 2, 256, [700, 65, 0, 31, 190]),
+def _looked_up(Hq, Hkv, lengths):
+    """Whether the launcher deals these packed requests by rank (else request by request, as a padded batch)."""
+    span = 32 * (4 // math.gcd(Hq // Hkv, 4))  # queries of a work item
+    tight = sum(lengths) // span + len(lengths)
+    return len(lengths) <= 256 and -(-max(lengths) // span) * len(lengths) > 2 * tight
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,lengths,looked_up", [
+    (16, 4, 128, [1], False),
+    (16, 4, 128, [33, 0, 1, 2048, 32, 64, 1000], True),            # equal and unequal tile counts, an empty request
+    (16, 4, 64, [(7 * i) % 91 for i in range(150)], False),        # 150 requests of like lengths
+    (16, 4, 64, [(7 * i) % 91 for i in range(150)] + [1500], True),  # more requests than lanes
+    (12, 4, 128, [300, 129, 127, 513], False),                     # one head per group: 128-query tiles, 12 head groups
+    (12, 4, 128, [1500, 60, 0, 31, 190], True),                    # 12 head groups: whole ones and a rest
+    (8, 8, 128, [1500, 60, 0, 31, 190, 5], True),                  # 8 head groups: one per XCD
+    (16, 16, 64, [1500, 60, 0, 31, 190, 5], True),                 # two per XCD
+    (9, 9, 64, [(31 * i) % 257 for i in range(65)], False),        # 9 head groups: one more than XCDs
+    (9, 9, 64, [1500, 60, 0, 31, 190, 5], True),
+    (4, 2, 64, [(13 * i) % 40 for i in range(255)] + [900], True),  # the most requests that are looked up
+    (4, 2, 64, [(13 * i) % 40 for i in range(256)] + [900], False),  # one more: dealt request by request
+    (4, 2, 64, [40 + (13 * i) % 40 for i in range(100)], False),   # like lengths: the same
+    (8, 2, 256, [700, 65, 0, 31, 190], True),
 ])
-def test_every_tile_of_packed_requests_is_computed(Hq, Hkv, D, lengths):
-    """The rank -> (request, tile) lookup of packed requests and the dealing of items over the XCDs cover every
-    row exactly once: each request's rows equal the request alone (key split off, as a packed call runs)."""
+def test_every_tile_of_packed_requests_is_computed(Hq, Hkv, D, lengths, looked_up):
+    """The rank -> (request, tile) lookup of packed requests and the dealing of items over the XCDs (fewer head groups
+    than XCDs, whole groups, both) cover every row exactly once: each request's rows equal the request alone (key split
+    off, as a packed call runs)."""
     from fastdecisions_amd.native_gqa_kernel import native_gqa_attention
+    assert _looked_up(Hq, Hkv, lengths) == looked_up
     cu = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
     T = int(cu[-1])
     announce(f"gqa packed {Hq}/{Hkv}x{D} n={len(lengths)} T={T}")
@@ -355,14 +371,16 @@ def test_head_dim_256_runs_whole_from_as_many_items_as_cus(B, Hq, Hkv, T):
     assert torch.equal(padded[:B], o)
 
 
-def test_launches_follow_the_current_stream_and_device():
-    """The raw handle is the current stream's, also inside a stream context, and the device guard enters
-    nothing on the current device."""
+def test_launches_follow_the_current_stream_and_device(monkeypatch):
+    """The raw handle is the current stream's, also inside a stream context; the device guard is nothing to enter on
+    the current device and the tensor's device (not entered here) where another is current."""
     from fastdecisions_amd import _lib
     dev = torch.device("cuda", torch.cuda.current_device())
     assert _lib.stream_handle(dev) == torch.cuda.current_stream(dev).cuda_stream
     side = torch.cuda.Stream()
     with torch.cuda.stream(side):
         assert _lib.stream_handle(dev) == side.cuda_stream
-    with _lib.on_device(dev):
-        assert torch.cuda.current_device() == dev.index
+    assert _lib.on_device(dev) is _lib._HERE
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: dev.index + 1)
+    guard = _lib.on_device(dev)
+    assert isinstance(guard, torch.cuda.device) and guard.idx == dev.index
