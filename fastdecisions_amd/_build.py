@@ -29,7 +29,6 @@ COMMON_FLAGS = [
     "-ffp-contract=off",
     "-fvisibility=hidden",
     "-Wall",
-    "-Wno-unused-function",
 ]
 DEVICE_FLAGS = [
     f"--offload-arch={OFFLOAD_ARCH}",

@@ -152,8 +152,6 @@ __device__ __forceinline__ int swz_v(int row) {
   return CR >= 16 ? 4 * (row & 3) : (2 * (row & 3)) & (CR - 1);
 }
 
-__device__ __forceinline__ bf16x8_t as_bf16x8(uint4 u) { return __builtin_bit_cast(bf16x8_t, u); }
-
 // Max / sum of a value over lanes l and l^32 (the two lane halves hold the two
 // 16-key halves of one query's scores).  v_permlane32_swap with the value in
 // both operands leaves this lane's value in one result and its partner's in
