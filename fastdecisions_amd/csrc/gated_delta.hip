@@ -18,7 +18,8 @@
 // Up to four launches, all on the caller's stream, intermediates in a
 // caller-provided workspace (fd_gated_delta_workspace_bytes):
 //   1. gd_chunk_table — packed requests only, one workgroup: chunk -> (first
-//      row, length), request -> first chunk.  A padded batch needs no table.
+//      row, length), request -> first chunk, the requests longest first.  A
+//      padded batch needs no table.
 //   2. gd_prep_kernel — one workgroup per (chunk, value head), chunk-parallel:
 //      l2norm, cumsum, the Gram and q.k tiles on bf16 MFMA (the normalised q/k
 //      are bf16 values, so these products are exact before fp32 accumulation),
@@ -708,7 +709,11 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
     // group of MFMAs.  The CU returns at most 64 B per cycle to all eight wavefronts
     // (the data return unit is busy 75 % of the pass), so a load issued with others
     // waits about 100 cycles in line; behind MFMAs that wait is theirs.
-    // sched_barrier keeps each in place.
+    // sched_barrier keeps each in place.  Spread so, the loads cost nothing: what
+    // sets the step are the LDS reads of the planes after its two barriers, 72 KB
+    // here and 66 KB by the output wavefronts (B=1, T=2048, copies for timing only,
+    // pass 40.5 us: no global loads at all 41.4; no plane reads here 38.4, by the
+    // outputs 37.0, by neither 27.9; no output work 37.4).
     int par = 0;  // the chunk's buffer of exponentials
     auto step = [&](const ChunkRegs& R, ChunkRegs& P) {
       // state at the chunk start: bf16 planes to LDS (B of w S and of the output's q S)
@@ -1164,10 +1169,12 @@ int gd_run(const void* q, const void* k, const void* v, const float* g, const vo
   const int64_t units = (nseq * v_heads + 7) / 8 * 8;  // (request, head) units, rounded up to the XCDs
   // Intermediates that do not fit the 256 MB memory-side cache beside q, k, v and the
   // output come from HBM, too late for loads two chunks ahead: long chains then fetch
-  // four chunks ahead into L2 (B=1, 16 heads: T=8192, 270 MB, 339 -> 282 us; T=7000,
-  // 232 MB, 248 -> 230; T=6000, 198 MB, 191.9 -> 188.8; T=4096, 135 MB, 123.6 ->
-  // 129.1; B=4, T=2048 236 -> 217).  Short chains pay for it (40 requests of 10 to
-  // 200 tokens: 164 -> 177 us).
+  // four chunks ahead into L2.  The line, 208 MiB = 218 MB, lies between the sizes that
+  // gain and lose (B=1, 16 heads: T=8192, 270 MB, 339 -> 282 us; T=7000, 232 MB, 248 ->
+  // 230; T=6000, 198 MB, 191.9 -> 188.8; T=4096, 135 MB, 123.6 -> 129.1; B=4, T=2048,
+  // 270 MB, 236 -> 217).  Short chains pay for it (40 requests of 10 to 200 tokens: 164
+  // -> 177 us), so the requests must have 24 chunks on average: the host knows no more
+  // of packed lengths.  One long request among many short ones runs without it.
   const dim3 state_grid(static_cast<unsigned>(units * kSlices));
   if (lay.ob > 208LL << 20 && nc >= 24 * nseq)
     hipLaunchKernelGGL(gd_state_kernel<true>, state_grid, dim3(kStateThreads), 0, s, a);
