@@ -60,6 +60,14 @@ constexpr int kD = 128;                // head_k_dim == head_v_dim
 constexpr int kSlice = 16;             // value columns per state workgroup
 constexpr int kSlices = kD / kSlice;   // state workgroups per (request, head)
 constexpr int kThreads = 256;
+// A's three planes in a chunk of GdArgs::aq (see aq_offset)
+constexpr int kAqPlane = 5 * 64 * 8 + 64;  // elements per plane (a multiple of 128 bytes)
+constexpr int kAqChunk = kC * kC * 2;      // elements per chunk
+// The order of packed requests lies behind the planes, an entry per chunk, so that it
+// takes no room of its own and the no-allocation scratch, a fixed size, takes every
+// call it took without it.  There are at least as many chunks as requests.
+constexpr int kOrderStep = kAqChunk / 2;   // int32 entries
+static_assert(3 * kAqPlane + 2 <= kAqChunk, "A's planes and an entry of the order fit in the space of the fp32 matrix");
 
 struct GdArgs {
   const uint16_t* q;
@@ -73,6 +81,10 @@ struct GdArgs {
   int32_t* row0;     // [nc]  first packed row of each chunk
   int32_t* len;      // [nc]  valid rows of each chunk (0 = unused)
   int32_t* first;    // [N+1] first chunk of each request
+  // requests, longest first: entry i at i * kOrderStep, behind A's planes in chunk i of aq.  (Formed
+  // from aq instead of held here, every call took 0.2 us longer: the arguments behind it then straddle
+  // one more line of the scalar loads at a workgroup's start.)
+  int32_t* order;
   float* gc;         // [Hv, nc, 3, 64]: e^{gc_t}, e^{gl - gc_t}, then e^{gl} 64 times (gl = gc of the last row)
   // q and A are stored in the state pass's output-wavefront operand order
   // (lane = 16 * g4 + c16): every load there reads 1-2 KiB contiguous
@@ -84,7 +96,7 @@ struct GdArgs {
                      // w split exactly into hi + mid + lo planes
   float* u;          // [Hv, nc, js 8, wv 4, lane 64, r 4]: u[16wv + 4g4 + r][16js + c16]
   uint16_t* aq;      // [Hv, nc, kAqChunk] bf16: planes hi, mid, lo (an exact split) of A[16rt + c16][32st + 8g4 + e],
-                     // e = 0..7 at aq_offset(rt, st, lane) of each plane; behind them order_entry
+                     // e = 0..7 at aq_offset(rt, st, lane) of each plane
   int hk, hv, nc, nseq;
   int varlen, seq_len, nct;  // packed requests (table) or a padded batch of nct chunks per sequence
   int beta_f32, l2norm;
@@ -172,22 +184,10 @@ __device__ __forceinline__ uint4 l2norm_row8(uint4 raw) {
 // request by a scan of their chunk counts, then every chunk's request by a
 // binary search, one chunk per thread (a thread per request that walked the
 // request's chunks took 12.8 us for requests of up to 8002 tokens; this takes 4.6).
-// order_entry lists the requests longest first, so that the state pass starts the
+// `order` lists the requests longest first, so that the state pass starts the
 // longest chains first (by counting, up to kTableThreads requests; more keep
 // their own order: their chains are many and short).
 constexpr int kTableThreads = 1024;
-
-// A's three planes in a chunk of GdArgs::aq (see aq_offset)
-constexpr int kAqPlane = 5 * 64 * 8 + 64;  // elements per plane (a multiple of 128 bytes)
-constexpr int kAqChunk = kC * kC * 2;      // elements per chunk
-static_assert(3 * kAqPlane + 2 <= kAqChunk, "the planes of A and an entry of `order` fit in the space of the fp32 matrix");
-// Entry `i` of the requests' order, longest first (packed requests): behind A's planes
-// in chunk i, so that the table takes no room of its own and the no-allocation
-// scratch, a fixed size, takes every call it took without it.  There are at least as
-// many chunks as requests.
-__device__ __forceinline__ int32_t* order_entry(const GdArgs& a, int i) {
-  return reinterpret_cast<int32_t*>(a.aq + static_cast<size_t>(i) * kAqChunk + 3 * kAqPlane);
-}
 
 __device__ __forceinline__ int request_rows(const int32_t* cu, int s, int total, int* start) {
   *start = min(max(cu[s], 0), total);
@@ -244,10 +244,10 @@ __global__ __launch_bounds__(kTableThreads) void gd_chunk_table(const int32_t* _
       if (s < nseq) {
         int rank = 0;
         for (int o = 0; o < nseq; ++o) rank += chunks[o] > n || (chunks[o] == n && o < s);
-        *order_entry(a, rank) = s;
+        a.order[static_cast<size_t>(rank) * kOrderStep] = s;
       }
     } else if (s < nseq) {
-      *order_entry(a, s) = s;
+      a.order[static_cast<size_t>(s) * kOrderStep] = s;
     }
     __syncthreads();
   }
@@ -636,7 +636,7 @@ __global__ __launch_bounds__(kStateThreads) void gd_state_kernel(GdArgs a) {
   if (unit >= a.nseq * a.hv) return;
   const int js = blockIdx.x / 8 % kSlices;
   const int h = unit % a.hv;
-  const int sq = a.varlen ? *order_entry(a, unit / a.hv) : unit / a.hv;
+  const int sq = a.varlen ? a.order[static_cast<size_t>(unit / a.hv) * kOrderStep] : unit / a.hv;
   int first, last;
   request_chunks(a, sq, &first, &last);
 
@@ -1146,6 +1146,7 @@ int gd_run(const void* q, const void* k, const void* v, const float* g, const vo
   a.w = reinterpret_cast<uint16_t*>(ws + lay.w);
   a.u = reinterpret_cast<float*>(ws + lay.u);
   a.aq = reinterpret_cast<uint16_t*>(ws + lay.aq);
+  a.order = reinterpret_cast<int32_t*>(a.aq + 3 * kAqPlane);
   a.hk = k_heads;
   a.hv = v_heads;
   a.nc = static_cast<int>(nc);
