@@ -33,9 +33,12 @@ def kernels(request):
 
 
 def test_a_wait_state_between_m0_and_the_copy_that_reads_it(kernels):
+    """M0 is written by the copies' asm alone (the compiler does not track it across one), never in the instruction
+    before the copy."""
     copies = 0
     for name, ins in kernels.items():
         for before, now in zip(ins, ins[1:]):
+            assert "m0" not in now[1] or (now[2] and now[0] == "s_mov_b32"), f"{name}: {now[3]}"
             if "_load_lds_" in now[0]:
                 copies += 1
                 assert before[1][:1] != ["m0"], f"{name}: {before[3]} directly before {now[3]}"
@@ -44,7 +47,7 @@ def test_a_wait_state_between_m0_and_the_copy_that_reads_it(kernels):
 
 def _registers(operand):
     kind, span = operand[0], operand[1:].strip("[]").split(":")
-    return {(kind, r) for r in range(int(span[0]), int(span[-1]) + 1)} if span[0].isdigit() else set()
+    return {(kind, r) for r in range(int(span[0]), int(span[-1]) + 1)}
 
 
 def test_no_asm_leaves_a_global_load_into_registers_in_flight(kernels):
